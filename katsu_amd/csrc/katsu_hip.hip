@@ -26,6 +26,7 @@
 #include "hostcopy.hpp"
 #include "pointwise.hpp"
 #include "smallc.hpp"
+#include "split.hpp"
 #include "stemdx.hpp"
 #include "tiny.hpp"
 
@@ -440,6 +441,33 @@ int gemm_rd_launch(const GemmArgs &g, hipStream_t st) {
     return launch_status();
 }
 
+// Whether a product runs on the bf16 matrix cores (split.hpp) rather than on
+// the float32 kernels here.  The float32 ones stay ahead where the matrix
+// cores are not what a call waits for (times on one MI355X, float32 / split):
+//   - K below 32: few products per stored output, and half of a split step is
+//     padding (4096 x 16 x 4096: 17.9 / 22.4 us);
+//   - aligned problems of 256 or more 32-tiles that leave CUs idle in 64-tiles
+//     (512^3: 6.9 / 8.0 us, 640^3: 11.0 / 12.7 us);
+//   - the register-direct plan's problems (1024^3: 20 us either way, its VJP
+//     37 / 39 us);
+//   - few tiles and a long sum, which the float32 plan splits over blocks and
+//     the split kernels only over a block's waves (64 x 8192 x 64: 9.3 / 50 us);
+//     equal near K = 900 (64 x 1000 x 64: 10.9 / 9.4 us; 16 x 1024 x 128: 8.6 /
+//     10.2).
+// Elsewhere the split ones win, by 1.1-1.7x on aligned problems (2048^3: 139 /
+// 109 us, 4096^3: 1041 / 640 us) and by more on others (1001 x 1531 x 777:
+// 59 / 26 us).  Operands of 1 GiB and more stay on the generic engine.
+constexpr int64_t kSplitMinK = 32, kSplitMaxKFewTiles = 900;
+
+bool gemm_on_split(const SplitProblem &p) {
+    if (!split_gemm_ok(p) || p.K < kSplitMinK) return false;
+    GemmArgs rd;
+    if (gemm_rd_plan(p.a, p.b, p.c, p.M, p.N, p.K, p.ta, p.tb, p.beta, &rd)) return false;
+    GemmFastPlan pl;
+    if (!gemm_fast_plan(p.a, p.b, p.c, p.M, p.N, p.K, p.ta, p.tb, p.beta, &pl)) return true;
+    return pl.T != 32 && (pl.splits == 1 || p.K <= kSplitMaxKFewTiles);
+}
+
 // The planned GEMM into c, with a fixed-order reduce of the partial slices
 // when K is split.
 bool gemm_fast(const float *a, const float *b, float *c, int64_t M, int64_t N, int64_t K, int ta,
@@ -504,6 +532,8 @@ int gemm_dev(const float *a, const float *b, float *c, size_t m, size_t n, size_
     if ((int64_t)m > kI32Max || (int64_t)n > kI32Max || (int64_t)k > kI32Max)
         return KATSU_E_INVALID;
     if (!a || !b) return KATSU_E_INVALID;
+    const SplitProblem sp{a, b, c, (int64_t)m, (int64_t)n, (int64_t)k, ta, tb, beta};
+    if (gemm_on_split(sp)) return split_gemm(sp, st);
     {
         int rc = KATSU_OK;
         if (gemm_fast(a, b, c, (int64_t)m, (int64_t)n, (int64_t)k, ta, tb, beta, st, &rc))
@@ -539,53 +569,59 @@ int matmul_vjp_dev(const float *a, const float *b, const float *g, float *da, fl
     const int64_t M = (int64_t)m, N = (int64_t)n, K = (int64_t)k;
     const bool apart = da && db && (da + M * K <= db || db + K * N <= da);
     if (apart && !empty && a && b && g) {
-        GemmArgs ra, rb;
-        if (gemm_rd_plan(g, b, da, M, K, N, 0, 1, beta_a, &ra) &&
-            gemm_rd_plan(a, g, db, K, N, M, 1, 0, beta_b, &rb) &&
-            (ra.tiles_m * ra.tiles_n) % 8 == 0) {
-            ra.c = da;
-            rb.c = db;
-            const int nb0 = ra.tiles_m * ra.tiles_n, nb1 = rb.tiles_m * rb.tiles_n;
-            if (KATSU_GEMM_RD_VJP_PAIR && nb0 == nb1) {
-                // One block per tile index: its dA tile, then its dB tile.
-                constexpr auto pk =
-                    gemm_rd_vjp_pair_kernel<kRdVjpKs, kRdVjpNkb, KATSU_GEMM_RD_VJP_D>;
+        const SplitProblem pa{g, b, da, M, K, N, 0, 1, beta_a}, pb{a, g, db, K, N, M, 1, 0, beta_b};
+        const bool sa = gemm_on_split(pa), sb = gemm_on_split(pb);
+        if (sa && sb) return split_gemm_vjp(pa, pb, st);
+        // One on each side: two launches, below.
+        if (!sa && !sb) {
+            GemmArgs ra, rb;
+            if (gemm_rd_plan(g, b, da, M, K, N, 0, 1, beta_a, &ra) &&
+                gemm_rd_plan(a, g, db, K, N, M, 1, 0, beta_b, &rb) &&
+                (ra.tiles_m * ra.tiles_n) % 8 == 0) {
+                ra.c = da;
+                rb.c = db;
+                const int nb0 = ra.tiles_m * ra.tiles_n, nb1 = rb.tiles_m * rb.tiles_n;
+                if (KATSU_GEMM_RD_VJP_PAIR && nb0 == nb1) {
+                    // One block per tile index: its dA tile, then its dB tile.
+                    constexpr auto pk =
+                        gemm_rd_vjp_pair_kernel<kRdVjpKs, kRdVjpNkb, KATSU_GEMM_RD_VJP_D>;
+                    constexpr size_t lds = kRdVjpKs * 64 * 64 * 4;
+                    const int rc = lds_optin<pk>(lds);
+                    if (rc != KATSU_OK) return rc;
+                    pk<<<dim3((unsigned)nb0), dim3(64 * kRdVjpKs), lds, st>>>(ra, rb);
+                    return launch_status();
+                }
+                constexpr auto kern =
+                    gemm_rd_vjp_kernel<kRdVjpKs, kRdVjpNkb, KATSU_GEMM_RD_VJP_D, KATSU_GEMM_RD_VJP_OCC>;
                 constexpr size_t lds = kRdVjpKs * 64 * 64 * 4;
-                const int rc = lds_optin<pk>(lds);
+                const int rc = lds_optin<kern>(lds);
                 if (rc != KATSU_OK) return rc;
-                pk<<<dim3((unsigned)nb0), dim3(64 * kRdVjpKs), lds, st>>>(ra, rb);
+                kern<<<dim3((unsigned)(nb0 + nb1)), dim3(64 * kRdVjpKs), lds, st>>>(ra, rb, nb0);
                 return launch_status();
             }
-            constexpr auto kern =
-                gemm_rd_vjp_kernel<kRdVjpKs, kRdVjpNkb, KATSU_GEMM_RD_VJP_D, KATSU_GEMM_RD_VJP_OCC>;
-            constexpr size_t lds = kRdVjpKs * 64 * 64 * 4;
-            const int rc = lds_optin<kern>(lds);
-            if (rc != KATSU_OK) return rc;
-            kern<<<dim3((unsigned)(nb0 + nb1)), dim3(64 * kRdVjpKs), lds, st>>>(ra, rb, nb0);
-            return launch_status();
-        }
-        GemmFastPlan pa, pb;
-        if (gemm_fast_plan(g, b, da, M, K, N, 0, 1, beta_a, &pa) &&
-            gemm_fast_plan(a, g, db, K, N, M, 1, 0, beta_b, &pb) && pa.T == pb.T &&
-            pa.splits == 1 && pb.splits == 1 && pa.blocks % 8 == 0 &&
-            pa.blocks + pb.blocks <= kI32Max) {
-            pa.g.c = da;
-            pb.g.c = db;
-            pa.g.split_stride = pb.g.split_stride = 0;
-            // Wave groups by the combined grid (two blocks per CU from the
-            // pair where each alone would take two groups): the k-sum order
-            // can then differ from the separate launches', within the f32
-            // bound and the same on every call.
-            const bool two = pa.blocks + pb.blocks < KATSU_GEMM_WG2_BELOW;
-            const int64_t b0 = pa.blocks, b1 = pb.blocks;
-            if (pa.T == 128)
-                return two ? gemm_vjp_launch<128, 128, 16, 2>(pa.g, pb.g, b0, b1, st)
-                           : gemm_vjp_launch<128, 128, 16, 1>(pa.g, pb.g, b0, b1, st);
-            if (pa.T == 64)
-                return two ? gemm_vjp_launch<64, 64, KATSU_GEMM_BK64, 2>(pa.g, pb.g, b0, b1, st)
-                           : gemm_vjp_launch<64, 64, KATSU_GEMM_BK64, 1>(pa.g, pb.g, b0, b1, st);
-            return two ? gemm_vjp_launch<32, 32, KATSU_GEMM_BK32, 2>(pa.g, pb.g, b0, b1, st)
-                       : gemm_vjp_launch<32, 32, KATSU_GEMM_BK32, 1>(pa.g, pb.g, b0, b1, st);
+            GemmFastPlan fa, fb;
+            if (gemm_fast_plan(g, b, da, M, K, N, 0, 1, beta_a, &fa) &&
+                gemm_fast_plan(a, g, db, K, N, M, 1, 0, beta_b, &fb) && fa.T == fb.T &&
+                fa.splits == 1 && fb.splits == 1 && fa.blocks % 8 == 0 &&
+                fa.blocks + fb.blocks <= kI32Max) {
+                fa.g.c = da;
+                fb.g.c = db;
+                fa.g.split_stride = fb.g.split_stride = 0;
+                // Wave groups by the combined grid (two blocks per CU from the
+                // pair where each alone would take two groups): the k-sum order
+                // can then differ from the separate launches', within the f32
+                // bound and the same on every call.
+                const bool two = fa.blocks + fb.blocks < KATSU_GEMM_WG2_BELOW;
+                const int64_t b0 = fa.blocks, b1 = fb.blocks;
+                if (fa.T == 128)
+                    return two ? gemm_vjp_launch<128, 128, 16, 2>(fa.g, fb.g, b0, b1, st)
+                               : gemm_vjp_launch<128, 128, 16, 1>(fa.g, fb.g, b0, b1, st);
+                if (fa.T == 64)
+                    return two ? gemm_vjp_launch<64, 64, KATSU_GEMM_BK64, 2>(fa.g, fb.g, b0, b1, st)
+                               : gemm_vjp_launch<64, 64, KATSU_GEMM_BK64, 1>(fa.g, fb.g, b0, b1, st);
+                return two ? gemm_vjp_launch<32, 32, KATSU_GEMM_BK32, 2>(fa.g, fb.g, b0, b1, st)
+                           : gemm_vjp_launch<32, 32, KATSU_GEMM_BK32, 1>(fa.g, fb.g, b0, b1, st);
+            }
         }
     }
     int rc = KATSU_OK;

@@ -1,0 +1,26 @@
+// split.hpp -- what the C ABI (katsu_hip.hip) calls of the split-bf16 kernels,
+// which are compiled apart from it (split.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace katsu {
+
+// One product C[M,N] = beta*C + op(A) op(B); row-major, packed.
+struct SplitProblem {
+    const float *a, *b;
+    float *c;
+    int64_t M, N, K;
+    int ta, tb;
+    float beta;
+};
+
+// Whether split_gemm takes p: operands below 1 GiB, the output below 2^31.
+bool split_gemm_ok(const SplitProblem &p);
+// Launches p; a katsu_status.
+int split_gemm(const SplitProblem &p, hipStream_t st);
+// Both in one launch: p with ta = 0, tb = 1 and q with ta = 1, tb = 0.
+int split_gemm_vjp(const SplitProblem &p, const SplitProblem &q, hipStream_t st);
+
+}  // namespace katsu

@@ -1,0 +1,75 @@
+// split3.hpp -- float32 products on the bf16 matrix cores: each operand is
+// written as the sum of three bf16 values, and a product as six of bf16 ones.
+//
+//   x = x0 + x1 + x2,  x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1
+//
+// (round to nearest).  A bf16 has 8 significant bits and the exponents of
+// float32, so |x1| <= 2^-9 |x|, |x2| <= 2^-18 |x|, both differences are exact
+// and nothing is left after x2: the split loses no bit of x (but below
+// 2^-133, where bf16 ends).  Of the nine products the kernels form six,
+//
+//   x0 y0 + (x0 y1 + x1 y0) + (x1 y1 + x0 y2 + x2 y0),
+//
+// each exact in float32; the three left out sum to at most 2^-26 |x y|, a
+// quarter of the rounding of one float32 product.
+//
+// v_mfma_f32_32x32x16_bf16 does 16x the FLOP per cycle of the float32
+// v_mfma_f32_16x16x4_f32, so six of them do the work of the float32 pipe in
+// 6/16 of its time: 333 TFLOP/s of float32 products at the 2.0 PFLOP/s that
+// a loop of nothing else reached, against 135-143 on the float32 pipe.
+//
+// Accumulation.  The instruction adds its 16 products to the accumulator
+// aligned to the largest term and keeps 2 bits below the accumulator's last
+// one (measured: 1 + 32 * 2^-26 is exact, 1 + 32 * 2^-27 is 1): a long sum
+// would lose the tails of terms of one sign.  The kernels therefore sum runs of
+// kFlush reduction steps from zero and add each run to a float32 total with
+// an ordinary addition, so that terms and accumulator stay near in size.
+//
+// Non-finite values: Inf - Inf in the split, or a value that rounds to Inf
+// in bf16, makes the result NaN; a finite result is never wrong.  Every
+// kernel tests its results and computes non-finite ones again in float32.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace katsu {
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
+
+// Eight floats as three vectors of eight bf16: 11 vector instructions a pair.
+// (The differences as two-term bf16 products on the packed pair are exact too
+// and take 7, but run slower beside the matrix instructions: 4096^3 in 687
+// against 632 us.)
+__device__ __forceinline__ void split3(const float (&x)[8], uintx4 (&p)[3]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const uint32_t h =
+                __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{a, b}, bf16x2));
+            p[q][i] = h;
+            if (q < 2) {
+                a -= __builtin_bit_cast(float, h << 16);
+                b -= __builtin_bit_cast(float, h & 0xffff0000u);
+            }
+        }
+    }
+}
+
+// The six products, smallest first.
+constexpr int kSplitA[6] = {2, 0, 1, 1, 0, 0};
+constexpr int kSplitB[6] = {0, 2, 1, 0, 1, 0};
+
+__device__ __forceinline__ floatx16 mfma32(uintx4 a, uintx4 b, floatx16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+}  // namespace katsu
