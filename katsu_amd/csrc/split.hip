@@ -3,9 +3,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <utility>
 
 #include "../../include/katsu_hip.h"
 #include "split.hpp"
+#include "splitconv.hpp"
 #include "splitgemm.hpp"
 
 namespace katsu {
@@ -13,6 +15,7 @@ namespace {
 
 constexpr int64_t kMaxElems = (int64_t)1 << 28;  // 1 GiB of floats
 constexpr int kCUs = 256;
+constexpr int kMaxLds = 160 * 1024;
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -176,6 +179,191 @@ int launch_vjp(const SplitProblem &p, const SplitProblem &q, hipStream_t st) {
     return status_of(hipGetLastError());
 }
 
+// ---------------------------------------------------------------------------
+// Convolutions.
+
+template <int FM, int FN, int WPX, int WKG, int TG, int XU>
+__global__ void __launch_bounds__(64 * WPX * WKG, 2) split_conv_kernel(const SplitConvArgs g) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    SplitConv<FM, FN, WPX, WKG, TG, XU>::run(g, lds, xcd_run(blockIdx.x, gridDim.x));
+}
+
+template <int FM, int FN, int WPX, int WKG, int TG, int XU>
+int conv_launch(const SplitConvArgs &g, int64_t blocks, hipStream_t st) {
+    using B = SplitConv<FM, FN, WPX, WKG, TG, XU>;
+    constexpr auto kern = split_conv_kernel<FM, FN, WPX, WKG, TG, XU>;
+    const int rc = lds_optin<kern>(kMaxLds);
+    if (rc != KATSU_OK) return rc;
+    kern<<<dim3((unsigned)blocks), dim3(B::kThreads), B::lds(g.slots), st>>>(g);
+    return status_of(hipGetLastError());
+}
+
+constexpr int kMaxStrip = 64;
+
+// Where a phase's tiles of BN pixels lie: strips of columns, pixels that tiles
+// do not cross the ends of, tiles, and input pixels of a tile in LDS.
+struct PhaseTiles {
+    int NS, SW, PW;
+    int64_t unit, utiles, tiles, slots;
+};
+
+PhaseTiles phase_tiles(const SplitPhase &p, int imgs, int st, int BN) {
+    PhaseTiles t;
+    t.NS = (int)cdiv(p.OW, kMaxStrip);
+    t.SW = (int)cdiv(p.OW, t.NS);
+    t.PW = (t.SW - 1) * st + p.Su;
+    const int64_t strip = (int64_t)p.OH * t.SW, strips = (int64_t)imgs * t.NS;
+    // Tiles end with their image's strip where that adds at most a tenth to
+    // them: the rows between two images then take no LDS.
+    const bool apart = cdiv(strip, BN) * BN * 10 <= strip * 11;
+    t.unit = apart ? strip : strip * strips;
+    t.utiles = cdiv(t.unit, BN);
+    t.tiles = t.utiles * (apart ? strips : 1);
+    const int64_t down = (t.SW - 1 + BN - 1) / t.SW;                 // output rows below the first
+    const int64_t cross = apart ? 0 : (p.OH - 1 + down) / p.OH;      // image ends among them
+    t.slots = (down * st + cross * std::max(0, p.Ru - st) + p.Ru) * t.PW;
+    return t;
+}
+
+// The block shapes, and the time of a chunk of 16 channels at 9 taps, in ns:
+// alone on a CU, and two blocks sharing it (measured on 3x3 layers: 512 ->
+// 512 channels at 7 x 7, 256 -> 256 at 14 x 14 and 64 -> 64 at 56 x 56, batch
+// 16-32).  The small tiles wait for their loads, the large ones approach the
+// matrix rate, so a layer takes the largest tile that still fills the GPU.
+struct ConvShape {
+    int FM, FN, WPX, WKG, TG;
+    double alone, shared;
+    constexpr int bm() const { return 32 * FM; }
+    constexpr int bn() const { return 32 * FN * WPX; }
+    constexpr int threads() const { return 64 * WPX * WKG; }
+};
+constexpr ConvShape kConvShapes[] = {{2, 2, 4, 1, 5, 9500, 14500},
+                                     {1, 2, 4, 1, 9, 5600, 7700},
+                                     {1, 1, 4, 2, 9, 3200, 4500},
+                                     {1, 1, 2, 4, 9, 2800, 3800}};
+constexpr int kNumConvShapes = 4;
+constexpr int kMaxXU = 8;
+
+template <int C>
+using ConvOf = SplitConv<kConvShapes[C].FM, kConvShapes[C].FN, kConvShapes[C].WPX,
+                         kConvShapes[C].WKG, kConvShapes[C].TG, 1>;
+template <int... C>
+constexpr int conv_lds_of(int c, int slots, std::integer_sequence<int, C...>) {
+    int v = 0;
+    ((c == C ? (void)(v = ConvOf<C>::lds(slots)) : (void)0), ...);
+    return v;
+}
+int conv_lds(int c, int slots) {
+    return conv_lds_of(c, slots, std::make_integer_sequence<int, kNumConvShapes>());
+}
+
+// The block shape of least estimated time, -1 if none takes the problem.
+int conv_pick(const SplitConvArgs &g) {
+    int best = -1;
+    double t_best = 0;
+    for (int c = 0; c < kNumConvShapes; ++c) {
+        const ConvShape &s = kConvShapes[c];
+        const int64_t tm = cdiv(g.CO, s.bm()), chunks = cdiv(g.CI, 16);
+        int64_t blocks = 0, slots = 0;
+        double taps = 0;
+        bool ok = true;
+        for (int i = 0; i < g.nphases; ++i) {
+            const SplitPhase &p = g.ph[i];
+            const PhaseTiles t = phase_tiles(p, g.imgs, g.st, s.bn());
+            const int64_t strips = (int64_t)g.imgs * t.NS;
+            ok = ok && strips * p.OH * t.SW + s.bn() < (int64_t)1 << 31 &&
+                 strips * ((p.OH - 1) * (int64_t)g.st + p.Ru) + 256 < (int64_t)1 << 31;
+            slots = std::max(slots, t.slots);
+            blocks += t.tiles * tm;
+            // Below five taps a chunk is bound by its loads.
+            taps += (double)t.tiles * tm * std::max(5, p.Ru * p.Su);
+        }
+        if (!ok || 2 * slots > kMaxXU * s.threads() || blocks >= (int64_t)1 << 31) continue;
+        const int lds = conv_lds(c, (int)slots);
+        if (lds > kMaxLds) continue;
+        // Registers of more than two blocks' waves fit for none of the shapes
+        // at their usual sizes.
+        const int64_t per_cu = lds <= kMaxLds / 2 ? 2 : 1;
+        const int64_t full = blocks / (kCUs * per_cu), rest = blocks - full * kCUs * per_cu;
+        const double round = per_cu == 2 ? s.shared : s.alone;
+        const double t = ((double)full * round + (rest > kCUs ? s.shared : rest ? s.alone : 0.)) *
+                         (double)chunks * taps / (double)blocks / 9.;
+        if (best < 0 || t < t_best) {
+            best = c;
+            t_best = t;
+        }
+    }
+    return best;
+}
+
+template <int C>
+int conv_go(SplitConvArgs &g, hipStream_t st) {
+    constexpr ConvShape S = kConvShapes[C];
+    g.slots = 0;
+    g.tiles_m = (int)cdiv(g.CO, S.bm());
+    int64_t tiles = 0;
+    for (int i = 0; i < g.nphases; ++i) {
+        SplitPhase &p = g.ph[i];
+        const PhaseTiles t = phase_tiles(p, g.imgs, g.st, S.bn());
+        p.NS = t.NS;
+        p.SW = t.SW;
+        p.PW = t.PW;
+        p.Hs = (p.OH - 1) * g.st + p.Ru;
+        p.taps = p.Ru * p.Su;
+        p.unit = (int)t.unit;
+        p.utiles = (int)t.utiles;
+        p.tile0 = (int)tiles;
+        p.by_sw = split_div(p.SW);
+        p.by_oh = split_div(p.OH);
+        p.by_ns = split_div(p.NS);
+        p.by_hs = split_div(p.Hs);
+        p.by_pw = split_div(p.PW);
+        p.by_su = split_div(p.Su);
+        p.by_ut = split_div(p.utiles);
+        g.slots = std::max(g.slots, (int)t.slots);
+        tiles += t.tiles;
+    }
+    const int64_t blocks = tiles * g.tiles_m;
+    // Input groups per thread.
+    const int units = 2 * g.slots;
+    if (units <= S.threads()) return conv_launch<S.FM, S.FN, S.WPX, S.WKG, S.TG, 1>(g, blocks, st);
+    if (units <= 2 * S.threads())
+        return conv_launch<S.FM, S.FN, S.WPX, S.WKG, S.TG, 2>(g, blocks, st);
+    if (units <= 4 * S.threads())
+        return conv_launch<S.FM, S.FN, S.WPX, S.WKG, S.TG, 4>(g, blocks, st);
+    return conv_launch<S.FM, S.FN, S.WPX, S.WKG, S.TG, kMaxXU>(g, blocks, st);
+}
+
+bool conv_run(SplitConvArgs &g, hipStream_t st, int *rc) {
+    switch (conv_pick(g)) {
+        case 0: *rc = conv_go<0>(g, st); return true;
+        case 1: *rc = conv_go<1>(g, st); return true;
+        case 2: *rc = conv_go<2>(g, st); return true;
+        case 3: *rc = conv_go<3>(g, st); return true;
+        default: return false;
+    }
+}
+
+bool layer_args(const SplitLayer &l, SplitConvArgs *g) {
+    const int64_t nx = (int64_t)l.N * l.C * l.H * l.W, ny = (int64_t)l.N * l.K * l.OH * l.OW;
+    const int64_t nw = (int64_t)l.K * l.C * l.R * l.S;
+    if (nx >= kMaxElems || ny >= kMaxElems || nw >= kMaxElems || l.st > 2) return false;
+    *g = SplitConvArgs{};
+    g->imgs = l.N;
+    g->w_bytes = (uint32_t)(nw * 4);
+    g->K = l.K;
+    g->C = l.C;
+    g->LH = l.H;
+    g->LW = l.W;
+    g->OH = l.OH;
+    g->OW = l.OW;
+    g->R = l.R;
+    g->S = l.S;
+    g->lst = l.st;
+    g->lpad = l.pad;
+    return true;
+}
+
 }  // namespace
 
 bool split_gemm_ok(const SplitProblem &p) {
@@ -203,6 +391,99 @@ int split_gemm_vjp(const SplitProblem &p, const SplitProblem &q, hipStream_t st)
         case 64: return launch_vjp<64>(p, q, st);
         default: return launch_vjp<32>(p, q, st);
     }
+}
+
+namespace {
+
+bool fwd_args(const SplitLayer &l, SplitConvArgs *out) {
+    SplitConvArgs &g = *out;
+    if (!layer_args(l, &g)) return false;
+    g.in_bytes = (uint32_t)((int64_t)l.N * l.C * l.H * l.W * 4);
+    g.CI = l.C;
+    g.CO = l.K;
+    g.H = l.H;
+    g.W = l.W;
+    g.HW = l.H * l.W;
+    g.st = l.st;
+    g.in_img = l.C * g.HW;
+    g.w_row = l.C * l.R * l.S;
+    g.w_red = l.R * l.S;
+    g.out_plane = l.OH * l.OW;
+    g.out_img = (int64_t)l.K * g.out_plane;
+    g.osy = l.OW;
+    g.osx = 1;
+    g.nphases = 1;
+    SplitPhase &p = g.ph[0];
+    p.OH = l.OH;
+    p.OW = l.OW;
+    p.pady = p.padx = l.pad;
+    p.Ru = l.R;
+    p.Su = l.S;
+    p.tu = l.S;
+    p.tv = 1;
+    return true;
+}
+
+bool dx_args(const SplitLayer &l, SplitConvArgs *out) {
+    SplitConvArgs &g = *out;
+    if (!layer_args(l, &g)) return false;
+    g.in_bytes = (uint32_t)((int64_t)l.N * l.K * l.OH * l.OW * 4);
+    g.CI = l.K;
+    g.CO = l.C;
+    g.H = l.OH;
+    g.W = l.OW;
+    g.HW = l.OH * l.OW;
+    g.st = 1;
+    g.in_img = l.K * g.HW;
+    g.w_row = l.R * l.S;
+    g.w_red = l.C * l.R * l.S;
+    g.out_plane = l.H * l.W;
+    g.out_img = (int64_t)l.C * g.out_plane;
+    g.osy = l.st * l.W;
+    g.osx = l.st;
+    g.dx = 1;
+    for (int py = 0; py < l.st; ++py)
+        for (int px = 0; px < l.st; ++px) {
+            if (py >= l.H || px >= l.W) continue;
+            // Input row py + st*a receives taps r = r0 + st*u from output row a + dy - u.
+            const int r0 = (py + l.pad) % l.st, s0 = (px + l.pad) % l.st;
+            if (r0 >= l.R || s0 >= l.S) return false;  // pixels no tap reaches
+            SplitPhase &p = g.ph[g.nphases++];
+            p.OH = (int)cdiv(l.H - py, l.st);
+            p.OW = (int)cdiv(l.W - px, l.st);
+            p.Ru = (int)cdiv(l.R - r0, l.st);
+            p.Su = (int)cdiv(l.S - s0, l.st);
+            p.pady = p.Ru - 1 - (py + l.pad - r0) / l.st;
+            p.padx = p.Su - 1 - (px + l.pad - s0) / l.st;
+            p.tu = -l.st * l.S;
+            p.tv = -l.st;
+            p.t0 = (r0 + l.st * (p.Ru - 1)) * l.S + s0 + l.st * (p.Su - 1);
+            p.o0 = py * l.W + px;
+        }
+    return true;
+}
+
+}  // namespace
+
+bool split_conv_fwd(const float *x, const float *w, float *y, const SplitLayer &l, hipStream_t st,
+                    int *rc) {
+    SplitConvArgs g;
+    if (!fwd_args(l, &g)) return false;
+    g.in = x;
+    g.w = w;
+    g.out = y;
+    return conv_run(g, st, rc);
+}
+
+bool split_conv_dx(const float *gy, const float *w, float *dx, const SplitLayer &l, float beta,
+                   hipStream_t st, int *rc) {
+    SplitConvArgs g;
+    if (!dx_args(l, &g)) return false;
+    g.in = gy;
+    g.w = w;
+    g.out = dx;
+    g.beta = beta;
+    return conv_run(g, st, rc);
 }
 
 }  // namespace katsu

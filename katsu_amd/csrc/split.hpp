@@ -23,4 +23,16 @@ int split_gemm(const SplitProblem &p, hipStream_t st);
 // Both in one launch: p with ta = 0, tb = 1 and q with ta = 1, tb = 0.
 int split_gemm_vjp(const SplitProblem &p, const SplitProblem &q, hipStream_t st);
 
+// A convolution layer: x [N][C][H][W], w [K][C][R][S], stride st, padding pad.
+struct SplitLayer {
+    int N, C, H, W, K, R, S, st, pad, OH, OW;
+};
+
+// The forward pass and the data gradient, dx = beta*dx + dX.  False: not a
+// layer these kernels take; otherwise *rc is the launch's katsu_status.
+bool split_conv_fwd(const float *x, const float *w, float *y, const SplitLayer &l, hipStream_t st,
+                    int *rc);
+bool split_conv_dx(const float *gy, const float *w, float *dx, const SplitLayer &l, float beta,
+                   hipStream_t st, int *rc);
+
 }  // namespace katsu

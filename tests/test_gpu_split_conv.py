@@ -1,0 +1,85 @@
+"""The convolution kernels on the bf16 matrix cores (csrc/splitconv.hpp) against float64.
+
+Layers at the edges of their tiles: images that share a tile and images that do not, strips of
+wide rows, channel counts off the chunks of 16 and the tiles of 32 and 64, filters of fewer and
+more taps than are staged together, both strides and all their phases, padding beyond the
+filter.  Bound: that of a float32 dot product in any order (tests/parity.py); what the split
+leaves out is at most a quarter of the rounding it counts per product."""
+import numpy as np
+import pytest
+
+from katsu_amd import synth
+from tests.parity import assert_within
+
+pytestmark = pytest.mark.gpu
+
+LAYERS = [  # x, w, stride, pad
+    ((3, 17, 7, 7), (33, 17, 3, 3), 1, 1),       # images share tiles, tails of every kind
+    ((2, 40, 29, 31), (70, 40, 3, 3), 1, 1),
+    ((1, 16, 20, 65), (32, 16, 3, 3), 1, 1),     # two strips of 33 and 32 columns
+    ((2, 9, 12, 130), (20, 9, 5, 5), 1, 2),      # three strips, 25 taps
+    ((32, 32, 40, 48), (64, 32, 3, 3), 1, 1),    # 64 x 256 and 32 x 256 tiles
+    ((9, 24, 56, 56), (96, 24, 2, 3), 1, 0),     # rectangular filter, no padding
+    ((2, 20, 13, 11), (18, 20, 3, 3), 1, 4),     # padding beyond the filter
+    ((2, 50, 33, 47), (30, 50, 7, 7), 2, 3),     # stride 2: four phases of 16, 12, 12, 9 taps
+    ((3, 36, 30, 29), (41, 36, 5, 5), 2, 2),
+    ((2, 48, 21, 70), (40, 48, 4, 4), 2, 1),     # even filter
+]
+
+
+def _ref(x, w, gy, stride, pad):
+    import torch
+    t = [torch.from_numpy(v.astype(np.float64)) for v in (x, w, gy)]
+    y = torch.nn.functional.conv2d(t[0], t[1], stride=stride, padding=pad)
+    dx = torch.nn.grad.conv2d_input(x.shape, t[1], t[2], stride=stride, padding=pad)
+    return y.numpy(), dx.numpy()
+
+
+@pytest.mark.parametrize("xs,ws,stride,pad", LAYERS)
+def test_split_conv(xs, ws, stride, pad):
+    import torch
+    from katsu_amd import ops
+    x, w = synth.uniform(1, xs), synth.he_normal(2, ws)
+    oh, ow = ((xs[i + 2] + 2 * pad - ws[i + 2]) // stride + 1 for i in (0, 1))
+    gy = synth.normal(3, (xs[0], ws[0], oh, ow))
+    dev = lambda a: torch.from_numpy(a).cuda()
+    y, dx = _ref(x, w, gy, stride, pad)
+    sy, sdx = _ref(np.abs(x), np.abs(w), np.abs(gy), stride, pad)
+    kf, kb = ws[1] * ws[2] * ws[3], ws[0] * ws[2] * ws[3]
+    got = ops.conv2d_forward(dev(x), dev(w), stride, pad)
+    assert_within(got.cpu().numpy(), y, sy, kf, "y")
+    got = ops.conv2d_backward_data(dev(gy), dev(w), xs, stride, pad)
+    assert_within(got.cpu().numpy(), dx, sdx, kb, "dX")
+    old = synth.uniform(4, xs)
+    acc = dev(old)
+    ops.conv2d_backward_data(dev(gy), dev(w), xs, stride, pad, out=acc, beta=1.0)
+    assert_within(acc.cpu().numpy(), old + dx, np.abs(old) + sdx, kb + 1, "dX, beta 1")
+    # Twice the same bits, and the same as the one-call backward's.
+    dx2, _ = ops.conv2d_backward(dev(x), dev(w), dev(gy), stride, pad)
+    assert torch.equal(dx2, got)
+
+
+@pytest.mark.parametrize("xs,ws,stride,pad", [LAYERS[0], LAYERS[3], LAYERS[8]])
+def test_split_conv_nonfinite(xs, ws, stride, pad):
+    """Inf and NaN reach exactly the outputs whose visited taps hold them (padding and the
+    filter's missing taps multiply nothing)."""
+    import torch
+    from katsu_amd import ops
+    x, w = synth.uniform(1, xs), synth.he_normal(2, ws)
+    x[0, 0, 0, 0], x[-1, 1, -1, -1], x[0, -1, xs[2] // 2, xs[3] // 2] = np.inf, -np.inf, np.nan
+    y = ops.conv2d_forward(torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda(), stride,
+                           pad).cpu().numpy()
+    xd, wd = x.astype(np.float64), w.astype(np.float64)
+    ref = np.zeros(y.shape)
+    h, wdt = xs[2], xs[3]
+    with np.errstate(invalid="ignore"):
+        for oy in range(y.shape[2]):
+            for ox in range(y.shape[3]):
+                y0, x0 = oy * stride - pad, ox * stride - pad
+                r = slice(max(0, -y0), min(ws[2], h - y0))
+                s = slice(max(0, -x0), min(ws[3], wdt - x0))
+                patch = xd[:, :, y0 + r.start:y0 + r.stop, x0 + s.start:x0 + s.stop]
+                ref[:, :, oy, ox] = (patch[:, None] * wd[None, :, :, r, s]).sum((2, 3, 4))
+    for mask in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(mask(y), mask(ref))
+    assert np.isfinite(ref).any() and not np.isfinite(ref).all()
