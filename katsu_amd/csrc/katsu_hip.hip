@@ -2305,11 +2305,12 @@ struct DwPlan {
     PwDwPlan pw;          // used when pw.ok (1x1, no padding)
     StemDwPlan stem;      // used when stem.ok
     TinyDwPlan tiny;      // used when tiny.ok
+    bool split;           // on the bf16 matrix cores (split.hpp)
 };
 
 template <class C>
 DwPlan dw_plan(const ConvDims &d) {
-    DwPlan pl;
+    DwPlan pl{};
     pl.tiles_m = (int)cdiv(d.K, C::BM);
     pl.tiles_n = (int)cdiv(d.CRS, C::BN);
     const int64_t tiles = (int64_t)pl.tiles_m * pl.tiles_n;
@@ -2331,6 +2332,25 @@ DwPlan dw_plan(const ConvDims &d) {
 
 DwPlan dw_plan_any(const ConvDims &d) {
     DirectDwPlan dp = direct_dw_plan_any(d);
+    // The direct kernel stays for stride 2 and where it shares the one-call
+    // backward's launch with a direct dX (64 -> 64 channels 3x3 at 56 x 56, batch
+    // 32: 134 us together; on the bf16 matrix cores 57 + 77).
+    DirectFwdProblem P;
+    DirectFwdPlan xp;
+    if (dp.ok && (d.st == 2 || (dx_as_forward(d, nullptr, nullptr, nullptr, 0.f, &P) &&
+                                P.CO >= FwdV::KT &&
+                                direct_fwd_plan<KATSU_FWD_VARIANT, 1>(P, &xp)))) {
+        DwPlan pl{};
+        pl.ws_bytes = dp.ws_bytes;
+        pl.direct = dp;
+        return pl;
+    }
+    if (!pw_ok(d) && !stem_dw_plan(d).ok && !tiny_dw_plan(d).ok) {
+        DwPlan pl{};
+        pl.ws_bytes = split_dw_bytes(split_layer(d));
+        pl.split = pl.ws_bytes > 0;
+        if (pl.split) return pl;
+    }
     if (dp.ok) {
         DwPlan pl{};
         pl.ws_bytes = dp.ws_bytes;
@@ -2429,6 +2449,7 @@ int conv_bwd_filter_dev(const float *x, const float *gy, float *dw, const katsu_
     float *wsp = nullptr;
     int rc = ws_take(src, pl.ws_bytes, st, &wsp);
     if (rc != KATSU_OK) return rc;
+    if (pl.split) return split_dw(x, gy, dw, split_layer(d), beta, wsp, st);
     if (pl.direct.ok) return direct_dw_launch(pl.direct, x, gy, dw, beta, wsp, st);
     if (pl.pw.ok) return pw_dw(x, gy, dw, d, pl.pw, beta, wsp, st);
     if (pl.stem.ok) return stem_dw_launch(pl.stem, x, gy, dw, beta, wsp, st);

@@ -8,6 +8,7 @@
 #include "../../include/katsu_hip.h"
 #include "split.hpp"
 #include "splitconv.hpp"
+#include "splitdw.hpp"
 #include "splitgemm.hpp"
 
 namespace katsu {
@@ -225,6 +226,25 @@ PhaseTiles phase_tiles(const SplitPhase &p, int imgs, int st, int BN) {
     return t;
 }
 
+// A phase's fields as phase_tiles lays it out; its first tile is 0.
+void phase_set(SplitPhase *p, const PhaseTiles &t, int imgs, int st) {
+    p->NS = t.NS;
+    p->SW = t.SW;
+    p->PW = t.PW;
+    p->Hs = (p->OH - 1) * st + p->Ru;
+    p->taps = p->Ru * p->Su;
+    p->unit = (int)t.unit;
+    p->utiles = (int)t.utiles;
+    p->npix = (int)((int64_t)imgs * t.NS * p->OH * t.SW);
+    p->by_sw = split_div(p->SW);
+    p->by_oh = split_div(p->OH);
+    p->by_ns = split_div(p->NS);
+    p->by_hs = split_div(p->Hs);
+    p->by_pw = split_div(p->PW);
+    p->by_su = split_div(p->Su);
+    p->by_ut = split_div(p->utiles);
+}
+
 // The block shapes, and the time of a chunk of 16 channels at 9 taps, in ns:
 // alone on a CU, and two blocks sharing it (measured on 3x3 layers: 512 ->
 // 512 channels at 7 x 7, 256 -> 256 at 14 x 14 and 64 -> 64 at 56 x 56, batch
@@ -305,21 +325,8 @@ int conv_go(SplitConvArgs &g, hipStream_t st) {
     for (int i = 0; i < g.nphases; ++i) {
         SplitPhase &p = g.ph[i];
         const PhaseTiles t = phase_tiles(p, g.imgs, g.st, S.bn());
-        p.NS = t.NS;
-        p.SW = t.SW;
-        p.PW = t.PW;
-        p.Hs = (p.OH - 1) * g.st + p.Ru;
-        p.taps = p.Ru * p.Su;
-        p.unit = (int)t.unit;
-        p.utiles = (int)t.utiles;
+        phase_set(&p, t, g.imgs, g.st);
         p.tile0 = (int)tiles;
-        p.by_sw = split_div(p.SW);
-        p.by_oh = split_div(p.OH);
-        p.by_ns = split_div(p.NS);
-        p.by_hs = split_div(p.Hs);
-        p.by_pw = split_div(p.PW);
-        p.by_su = split_div(p.Su);
-        p.by_ut = split_div(p.utiles);
         g.slots = std::max(g.slots, (int)t.slots);
         tiles += t.tiles;
     }
@@ -484,6 +491,110 @@ bool split_conv_dx(const float *gy, const float *w, float *dx, const SplitLayer 
     g.out = dx;
     g.beta = beta;
     return conv_run(g, st, rc);
+}
+
+namespace {
+
+template <int XU>
+__global__ void __launch_bounds__(768, 3) split_dw_kernel(const SplitDwArgs g) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    SplitDw<XU>::run(g, lds, xcd_run(blockIdx.x, gridDim.x));
+}
+
+// Partial sums in the workspace: at most the 37.7 MB that the library's other
+// plans need, which the static array of the allocation-free backward holds.
+constexpr int64_t kMaxPartBytes = 37700000;
+
+bool dw_args(const SplitLayer &l, SplitDwArgs *out) {
+    using B = SplitDw<1>;
+    SplitConvArgs f;
+    if (!fwd_args(l, &f)) return false;
+    SplitDwArgs &g = *out;
+    g = SplitDwArgs{};
+    g.x_bytes = f.in_bytes;
+    g.g_bytes = (uint32_t)((int64_t)l.N * l.K * l.OH * l.OW * 4);
+    g.C = l.C;
+    g.K = l.K;
+    g.H = l.H;
+    g.W = l.W;
+    g.HW = l.H * l.W;
+    g.OHW = l.OH * l.OW;
+    g.st = l.st;
+    g.imgs = l.N;
+    g.R = l.R;
+    g.S = l.S;
+    g.pad = l.pad;
+    g.ph = f.ph[0];
+    const PhaseTiles t = phase_tiles(g.ph, l.N, l.st, B::P);
+    const int64_t npix = (int64_t)l.N * t.NS * l.OH * t.SW;
+    if (npix + 2 * B::P >= (int64_t)1 << 31 ||
+        (int64_t)l.N * t.NS * ((l.OH - 1) * (int64_t)l.st + l.R) + 256 >= (int64_t)1 << 31)
+        return false;
+    if (t.slots * (B::BC / 8) > 4 * B::kThreads || B::lds((int)t.slots) > kMaxLds) return false;
+    phase_set(&g.ph, t, l.N, l.st);
+    g.slots = (int)t.slots;
+    g.tiles = (int)t.tiles;
+    g.tiles_k = (int)cdiv(l.K, B::BK);
+    g.tiles_c = (int)cdiv(l.C, B::BC);
+    g.sets = (int)cdiv(g.ph.taps, 9);
+    g.run_stride = ((int64_t)l.K * l.C * g.ph.taps + 3) / 4 * 4;
+    // One block per CU, each with at least two tiles.
+    const int64_t blocks = (int64_t)g.tiles_k * g.tiles_c * g.sets;
+    int64_t runs = std::max<int64_t>(1, kCUs / blocks);
+    runs = std::min(runs, std::max<int64_t>(1, g.tiles / 2));
+    runs = std::min(runs, std::max<int64_t>(1, kMaxPartBytes / (g.run_stride * 4)));
+    if (g.run_stride * 4 > kMaxPartBytes) return false;
+    g.per_run = (int)cdiv(g.tiles, runs);
+    g.runs = (int)cdiv(g.tiles, g.per_run);
+    return blocks * g.runs < (int64_t)1 << 31;
+}
+
+template <int XU>
+int dw_launch(const SplitDwArgs &g, hipStream_t st) {
+    constexpr auto kern = split_dw_kernel<XU>;
+    const int rc = lds_optin<kern>(kMaxLds);
+    if (rc != KATSU_OK) return rc;
+    const int64_t blocks = (int64_t)g.tiles_k * g.tiles_c * g.sets * g.runs;
+    kern<<<dim3((unsigned)blocks), dim3(SplitDw<XU>::kThreads), SplitDw<XU>::lds(g.slots), st>>>(g);
+    return status_of(hipGetLastError());
+}
+
+}  // namespace
+
+size_t split_dw_bytes(const SplitLayer &l) {
+    SplitDwArgs g;
+    // Below 1.5 GFLOP of products, its tiles' padding counted, the launch, the
+    // first loads and the partial sums' reduction outweigh the matrix rate (one
+    // image of 64 -> 64 channels, 0.23 GFLOP: 31 us against 21; 128 -> 128 at
+    // 28 x 28, batch 8, 1.85 GFLOP: 38 against 45).  So do half-empty tiles
+    // (13 -> 15 channels 5x5: 266 against 205).
+    const double flops = 2. * l.N * l.OH * l.OW * l.K * l.C * l.R * l.S;
+    const double fill = (double)l.K * l.C / ((double)cdiv(l.K, 64) * 64 * cdiv(l.C, 32) * 32);
+    if (flops < 1.5e9 || fill < 0.5) return 0;
+    return dw_args(l, &g) ? (size_t)(g.runs * g.run_stride) * sizeof(float) : 0;
+}
+
+int split_dw(const float *x, const float *gy, float *dw, const SplitLayer &l, float beta, float *ws,
+             hipStream_t st) {
+    SplitDwArgs g;
+    if (!dw_args(l, &g)) return KATSU_E_INVALID;
+    g.x = x;
+    g.g = gy;
+    g.part = ws;
+    const int units = g.slots * (SplitDw<1>::BC / 8), th = SplitDw<1>::kThreads;
+    const int rc = units <= th ? dw_launch<1>(g, st)
+                   : units <= 2 * th ? dw_launch<2>(g, st) : dw_launch<4>(g, st);
+    if (rc != KATSU_OK) return rc;
+    const int64_t n = (int64_t)l.K * l.C * g.ph.taps;
+    // Few runs: small blocks, whose threads then all have one to read.
+    const dim3 blocks((unsigned)cdiv(n, 64));
+    if (g.runs <= 32)
+        split_dw_reduce<4><<<blocks, dim3(256), 0, st>>>(ws, dw, g.run_stride, g.runs, l.K * l.C,
+                                                         g.ph.taps, beta);
+    else
+        split_dw_reduce<16><<<blocks, dim3(1024), 0, st>>>(ws, dw, g.run_stride, g.runs, l.K * l.C,
+                                                           g.ph.taps, beta);
+    return status_of(hipGetLastError());
 }
 
 }  // namespace katsu

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace katsu {
@@ -34,5 +35,11 @@ bool split_conv_fwd(const float *x, const float *w, float *y, const SplitLayer &
                     int *rc);
 bool split_conv_dx(const float *gy, const float *w, float *dx, const SplitLayer &l, float beta,
                    hipStream_t st, int *rc);
+
+// The filter gradient, dw = beta*dw + dW.  split_dw_bytes: the workspace it
+// needs, 0 if it does not take the layer.
+size_t split_dw_bytes(const SplitLayer &l);
+int split_dw(const float *x, const float *gy, float *dw, const SplitLayer &l, float beta, float *ws,
+             hipStream_t st);
 
 }  // namespace katsu

@@ -83,3 +83,44 @@ def test_split_conv_nonfinite(xs, ws, stride, pad):
     for mask in (np.isnan, np.isposinf, np.isneginf):
         assert np.array_equal(mask(y), mask(ref))
     assert np.isfinite(ref).any() and not np.isfinite(ref).all()
+
+
+DW_LAYERS = [  # x, w, stride, pad: 1.5 GFLOP or more, so that the split kernel takes them
+    ((30, 96, 20, 20), (128, 96, 3, 3), 1, 1),   # whole images
+    ((40, 160, 14, 14), (130, 160, 3, 3), 1, 1),  # tiles across images, channel tail
+    ((3, 40, 90, 130), (60, 40, 5, 5), 1, 2),    # strips, three sets of taps
+    ((8, 64, 30, 33), (64, 64, 7, 7), 1, 3),
+]
+
+
+@pytest.mark.parametrize("xs,ws,stride,pad", DW_LAYERS)
+def test_split_dw(xs, ws, stride, pad):
+    """Sampled exact sums, the corners among them; the same bits twice and in the one-call
+    backward; beta = 1; and Inf and NaN in the sums that hold them only."""
+    import torch
+    from katsu_amd import ops
+    from tests.parity import random_samples, sample_dw
+    x, w = synth.uniform(1, xs), synth.he_normal(2, ws)
+    oh, ow = ((xs[i + 2] + 2 * pad - ws[i + 2]) // stride + 1 for i in (0, 1))
+    gy = synth.normal(3, (xs[0], ws[0], oh, ow))
+    dev = lambda a: torch.from_numpy(a).cuda()
+    at = random_samples(ws, 200, 5) + [(0, 0, 0, 0), tuple(d - 1 for d in ws)]
+    pick = lambda t: np.array([t[i] for i in at])
+    ref, sabs = sample_dw(x, gy, ws, stride, pad, at)
+    n = xs[0] * oh * ow
+    dw = ops.conv2d_backward_filter(dev(x), dev(gy), ws, stride, pad)
+    assert_within(pick(dw.cpu().numpy()), ref, sabs, n, "dW")
+    _, dw2 = ops.conv2d_backward(dev(x), dev(w), dev(gy), stride, pad)
+    assert torch.equal(dw, dw2)
+    old = synth.uniform(4, ws)
+    acc = dev(old)
+    ops.conv2d_backward_filter(dev(x), dev(gy), ws, stride, pad, out=acc, beta=1.0)
+    assert torch.equal(acc, dev(old) + dw)
+    # One pixel of one input channel, at a corner: only the taps that reach it.
+    x[1, 2, 0, 0] = np.inf
+    gy[1, 3, 0, 0] = 0.5
+    got = ops.conv2d_backward_filter(dev(x), dev(gy), ws, stride, pad).cpu().numpy()
+    bad = ~np.isfinite(got)
+    reach = np.zeros(ws[2:], bool)
+    reach[max(0, pad - oh + 1):pad + 1, max(0, pad - ow + 1):pad + 1] = True
+    assert np.array_equal(bad[3, 2], reach) and not np.delete(bad, 2, axis=1).any()
