@@ -5,8 +5,8 @@
 //
 // (round to nearest).  A bf16 has 8 significant bits and the exponents of
 // float32, so |x1| <= 2^-9 |x|, |x2| <= 2^-18 |x|, both differences are exact
-// and nothing is left after x2: the split loses no bit of x (but below
-// 2^-133, where bf16 ends).  Of the nine products the kernels form six,
+// and nothing is left after x2: the split loses no bit of x (but those below
+// 2^-133, where bf16 ends: an x below 2^-109 in size can lose some).  Of the nine products the kernels form six,
 //
 //   x0 y0 + (x0 y1 + x1 y0) + (x1 y1 + x0 y2 + x2 y0),
 //

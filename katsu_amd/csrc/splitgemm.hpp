@@ -31,7 +31,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t split_rsrc(const float *p, uin
                                              0x00020000);
 }
 // Floats at byte offset off (per lane) + so (the wave's): one, or eight in a
-// row.  A buffer load needs 4-byte alignment only, whatever its width.
+// row.  A buffer load needs 4-byte alignment only, whatever its width.  The
+// range check of an unswizzled buffer counts both parts and does not wrap
+// (1024 bytes described, off 0..504: so = 768 returns the first 256 bytes' lanes
+// and zeros, so = 24000 zeros), so a channel or k past the end reads zero.
 __device__ __forceinline__ float load1(__amdgpu_buffer_rsrc_t r, int off, int so) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, so, 0));
 }
