@@ -567,7 +567,8 @@ size_t split_dw_bytes(const SplitLayer &l) {
     // first loads and the partial sums' reduction outweigh the matrix rate (one
     // image of 64 -> 64 channels, 0.23 GFLOP: 31 us against 21; 128 -> 128 at
     // 28 x 28, batch 8, 1.85 GFLOP: 38 against 45).  So do half-empty tiles
-    // (13 -> 15 channels 5x5: 266 against 205).
+    // (13 -> 15 channels 5x5: 266 against 205; 45 -> 83 channels 5x5, 46% full:
+    // forward + backward 155 against 145).
     const double flops = 2. * l.N * l.OH * l.OW * l.K * l.C * l.R * l.S;
     const double fill = (double)l.K * l.C / ((double)cdiv(l.K, 64) * 64 * cdiv(l.C, 32) * 32);
     if (flops < 1.5e9 || fill < 0.5) return 0;
