@@ -1,12 +1,18 @@
 // split3.hpp -- float32 products on the bf16 matrix cores: each operand is
 // written as the sum of three bf16 values, and a product as six of bf16 ones.
 //
-//   x = x0 + x1 + x2,  x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1
+//   2^16 x = x0 + x1 + x2,  x0 = bf16(2^16 x), x1 = bf16(2^16 x - x0), x2 = the rest
 //
 // (round to nearest).  A bf16 has 8 significant bits and the exponents of
-// float32, so |x1| <= 2^-9 |x|, |x2| <= 2^-18 |x|, both differences are exact
-// and nothing is left after x2: the split loses no bit of x (but those below
-// 2^-133, where bf16 ends: an x below 2^-109 in size can lose some).  Of the nine products the kernels form six,
+// float32, so |x1| <= 2^-9 |x0|, |x2| <= 2^-18 |x0|, both differences are exact
+// and nothing is left after x2: the split loses no bit of x.  The factor keeps
+// that so for the smallest x: a bf16 ends at 2^-133, a float32 at 2^-149, and
+// without it operands below 2^-109 (1.5e-33) lost bits, those below 2^-134 all
+// of them.  Sums are multiplied by 2^-32, which is exact above 2^-126.
+// Operands of 2^112 and sums of 2^96 overflow in turn, and take the
+// way of the non-finite ones below.
+//
+// Of the nine products the kernels form six,
 //
 //   x0 y0 + (x0 y1 + x1 y0) + (x1 y1 + x0 y2 + x2 y0),
 //
@@ -25,9 +31,10 @@
 // kFlush reduction steps from zero and add each run to a float32 total with
 // an ordinary addition, so that terms and accumulator stay near in size.
 //
-// Non-finite values: Inf - Inf in the split, or a value that rounds to Inf
-// in bf16, makes the result NaN; a finite result is never wrong.  Every
-// kernel tests its results and computes non-finite ones again in float32.
+// Non-finite values: Inf - Inf in the split, or a value that overflows when it
+// is scaled or rounded to bf16, makes the sum NaN or Inf; a finite sum holds
+// finite products only.  Every kernel tests its sums and computes non-finite
+// ones again in float32.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -42,14 +49,17 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 
-// Eight floats as three vectors of eight bf16: 11 vector instructions a pair.
+constexpr float kSplitScale = 0x1p16f;     // of an operand
+constexpr float kSplitUnscale = 0x1p-32f;  // of a sum
+
+// Eight floats as three vectors of eight bf16: 13 vector instructions a pair.
 // (The differences as two-term bf16 products on the packed pair are exact too
 // and take 7, but run slower beside the matrix instructions: 4096^3 in 687
 // against 632 us.)
 __device__ __forceinline__ void split3(const float (&x)[8], uintx4 (&p)[3]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        float a = x[2 * i], b = x[2 * i + 1];
+        float a = kSplitScale * x[2 * i], b = kSplitScale * x[2 * i + 1];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             const uint32_t h =

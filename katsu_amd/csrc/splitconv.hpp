@@ -300,7 +300,10 @@ struct SplitConv {
 #pragma unroll
             for (int b = 0; b < FN; ++b)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) bad |= !__builtin_isfinite(tot[a][b][v]);
+                for (int v = 0; v < 16; ++v) {
+                    bad |= !__builtin_isfinite(tot[a][b][v]);
+                    tot[a][b][v] *= kSplitUnscale;
+                }
         const bool redo = __any(bad);
         // The wave's own part of the LDS, which nothing reads any more: the
         // rare recomputation then is a loop over values in memory, outside the

@@ -255,7 +255,10 @@ struct SplitDw {
 #pragma unroll
         for (int i = 0; i < TPW; ++i)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) bad |= !__builtin_isfinite(tot[i][v]);
+            for (int v = 0; v < 16; ++v) {
+                bad |= !__builtin_isfinite(tot[i][v]);
+                tot[i][v] *= kSplitUnscale;
+            }
         if (__any(bad)) {
             const int un0 = P0.by_ut.div(tile0), un1 = P0.by_ut.div(tile1);
             const int q0 = un0 * P0.unit + (tile0 - un0 * P0.utiles) * P;

@@ -323,7 +323,8 @@ struct SplitGemm {
                     const int i = i0 + a * 32 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
                     if (i >= g.M) continue;
                     float *c = g.c + (int64_t)i * g.ldc + j;
-                    *c = g.beta == 0.f ? tot[a][b][v] : g.beta * *c + tot[a][b][v];
+                    const float sum = kSplitUnscale * tot[a][b][v];
+                    *c = g.beta == 0.f ? sum : g.beta * *c + sum;
                 }
         }
     }
@@ -466,6 +467,7 @@ struct SplitGemmRd {
 #pragma unroll
             for (int w = 1; w < WAVES; ++w) out[e] += s[w * BM * BN + tid + e * kThreads];
             bad |= !__builtin_isfinite(out[e]);
+            out[e] *= kSplitUnscale;
         }
         if (__syncthreads_or(bad)) {
             split_again<BM, BN, kThreads, TA, TB>(g, i0, j0, lds);

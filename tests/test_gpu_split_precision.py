@@ -1,0 +1,66 @@
+"""What the three bf16 values and the six products of csrc/split3.hpp must keep of a float32.
+
+The bound of tests/parity.py is relative to each operand, whatever its size: it also holds
+where an operand is so small that bf16 values of it would be subnormal, or so large that a
+scaled one overflows."""
+import numpy as np
+import pytest
+
+from katsu_amd import synth
+from tests.parity import assert_within, random_samples, sample_dw, sample_dx, sample_fwd
+from tests.test_gpu_split_conv import DW_LAYERS, LAYERS
+from tests.test_gpu_split_gemm import SHAPES, _dev
+
+pytestmark = pytest.mark.gpu
+
+# Operand sizes: normal floats near the smallest, subnormal ones, and large ones, with a
+# partner that brings the products back to ordinary numbers.
+SCALES = [(1e-34, 1e15), (1e-37, 1e20), (1e20, 1e-37), (1e-40, 1e25), (1e-18, 1e-18),
+          (1e33, 1e-30), (1e20, 1e14)]
+
+
+def _scaled(seed, shape, s):
+    return (synth.uniform(seed, shape).astype(np.float64) * s).astype(np.float32)
+
+
+def _pick(t, at):
+    v = t.cpu().numpy()
+    return np.array([v[i] for i in at])
+
+
+@pytest.mark.parametrize("m,k,n", SHAPES[::2] + SHAPES[5:6] + SHAPES[7:])
+@pytest.mark.parametrize("s,t", SCALES)
+def test_gemm_operand_scales(m, k, n, s, t):
+    from katsu_amd import ops
+    a, b = _scaled(11, (m, k), s), _scaled(12, (k, n), t)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    c = ops.gemm(_dev(a), _dev(b), m, n, k).cpu().numpy()
+    assert_within(c, a64 @ b64, np.abs(a64) @ np.abs(b64), k, "C")
+
+
+@pytest.mark.parametrize("xs,ws,stride,pad", [LAYERS[0], LAYERS[4], LAYERS[7]])
+@pytest.mark.parametrize("s,t", SCALES)
+def test_conv_operand_scales(xs, ws, stride, pad, s, t):
+    from katsu_amd import ops
+    x, w = _scaled(1, xs, s), _scaled(2, ws, t)
+    oh, ow = ((xs[i + 2] + 2 * pad - ws[i + 2]) // stride + 1 for i in (0, 1))
+    gs = (xs[0], ws[0], oh, ow)
+    gy = _scaled(3, gs, s)
+    y = ops.conv2d_forward(_dev(x), _dev(w), stride, pad)
+    at = random_samples(gs, 300, 7)
+    assert_within(_pick(y, at), *sample_fwd(x, w, stride, pad, at), ws[1] * ws[2] * ws[3], "y")
+    dx = ops.conv2d_backward_data(_dev(gy), _dev(w), xs, stride, pad)
+    at = random_samples(xs, 300, 8)
+    assert_within(_pick(dx, at), *sample_dx(gy, w, xs, stride, pad, at), ws[0] * ws[2] * ws[3],
+                  "dX")
+
+
+@pytest.mark.parametrize("s,t", SCALES)
+def test_dw_operand_scales(s, t):
+    from katsu_amd import ops
+    xs, ws, stride, pad = DW_LAYERS[1]
+    oh, ow = ((xs[i + 2] + 2 * pad - ws[i + 2]) // stride + 1 for i in (0, 1))
+    x, gy = _scaled(1, xs, s), _scaled(3, (xs[0], ws[0], oh, ow), t)
+    dw = ops.conv2d_backward_filter(_dev(x), _dev(gy), ws, stride, pad)
+    at = random_samples(ws, 200, 5)
+    assert_within(_pick(dw, at), *sample_dw(x, gy, ws, stride, pad, at), xs[0] * oh * ow, "dW")
