@@ -14,7 +14,8 @@
 namespace katsu {
 namespace {
 
-constexpr int64_t kMaxElems = (int64_t)1 << 28;  // 1 GiB of floats
+constexpr int64_t kMaxElems = (int64_t)1 << 28;   // 1 GiB of floats
+constexpr int64_t kMaxOffset = (int64_t)1 << 29;  // floats below 2^31 bytes
 constexpr int kCUs = 256;
 constexpr int kMaxLds = 160 * 1024;
 
@@ -355,6 +356,13 @@ bool layer_args(const SplitLayer &l, SplitConvArgs *g) {
     const int64_t nx = (int64_t)l.N * l.C * l.H * l.W, ny = (int64_t)l.N * l.K * l.OH * l.OW;
     const int64_t nw = (int64_t)l.K * l.C * l.R * l.S;
     if (nx >= kMaxElems || ny >= kMaxElems || nw >= kMaxElems || l.st > 2) return false;
+    // The kernels' scalar offsets reach the end of a chunk of 16 channels, and in
+    // the filter of the one after it: few channels of large planes (5 of 6000 x
+    // 6000) would pass the 2^31 bytes that load1 allows.
+    const int64_t cs = cdiv(l.C, 16) * 16, ks = cdiv(l.K, 16) * 16;
+    if (cs * l.H * l.W >= kMaxOffset || ks * l.OH * l.OW >= kMaxOffset ||
+        (ks + 16) * l.C * l.R * l.S >= kMaxOffset || (cs + 16) * l.R * l.S >= kMaxOffset)
+        return false;
     *g = SplitConvArgs{};
     g->imgs = l.N;
     g->w_bytes = (uint32_t)(nw * 4);

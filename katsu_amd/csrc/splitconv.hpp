@@ -147,7 +147,8 @@ struct SplitConv {
                 const int iy = Y - im * P.Hs - P.pady;
                 const int ix = (im - n * P.NS) * P.SW * st + col - P.padx;
                 xdst[e] = cg * xplane + slot * 16;
-                if (n < g.imgs && (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W)
+                if (n < g.imgs && (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W &&
+                    cg * 8 < g.CI)
                     xoff[e] = (n * g.in_img + cg * 8 * g.HW + iy * g.W + ix) * 4;
             }
         }
@@ -185,12 +186,11 @@ struct SplitConv {
         // product that is then not finite is computed again like any other.
         // (Lanes' offsets selected in the last chunk instead: forward + backward
         // of 64 -> 64 channels 3x3 at 56 x 56, batch 32, 189 -> 221 us.)
-        auto load_x = [&](int c0) {
+        auto load_x = [&](int so) {
 #pragma unroll
             for (int e = 0; e < XU; ++e)
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    xr[e][i] = load1(rin, xoff[e], (c0 + i) * g.HW * 4);
+                for (int i = 0; i < 8; ++i) xr[e][i] = load1(rin, xoff[e], so + i * g.HW * 4);
         };
         const int su = P.Su, taps = P.taps, pw = P.PW, wt0 = P.t0, wtu = P.tu, wtv = P.tv;
         const SplitDiv by_su = P.by_su;
@@ -234,7 +234,8 @@ struct SplitConv {
                 __syncthreads();
                 const bool last = gt + 1 == groups;
                 load_w((last ? c + 1 : c) * 16, last ? 0 : (gt + 1) * TG);
-                if (gt == 0) load_x((c + 1) * 16);
+                // After the last chunk: out of range, which reads no memory.
+                if (gt == 0) load_x(c + 1 < chunks ? (c + 1) * 16 * g.HW * 4 : kSplitEnd);
                 __builtin_amdgcn_sched_barrier(kSchedNoVmem);
                 const int t0 = gt * TG, nt = min(TG, taps - t0);
                 for (int tl = wkg; tl < nt; tl += WKG) {

@@ -124,7 +124,7 @@ struct SplitDw {
             const int cg = u / g.slots, slot = u - cg * g.slots;
             xrow[e] = P0.by_pw.div(slot);
             xcol[e] = slot - xrow[e] * P0.PW - P0.padx;
-            xcg[e] = (c0 + cg * 8) * g.HW;
+            xcg[e] = cg < BC / 8 && c0 + cg * 8 < g.C ? (c0 + cg * 8) * g.HW : -1;
             xdst[e] = cg < BC / 8 ? cg * xp + slot * 16 : -1;
         }
 
@@ -142,20 +142,23 @@ struct SplitDw {
             const bool in = q < qend && ox < P0.OW;
             const int Y = im * P0.Hs + y * g.st;
             slot_next = in ? ((Y - Y0) * P0.PW + xs * g.st) * 16 : 0;
-            const int go = in ? (n * g.K * g.OHW + y * P0.OW + ox + (k0 + gk * 8) * g.OHW) * 4
-                              : kSplitOOB;
+            // Groups that begin past the last channel read zeros; the others' end
+            // reads the next image's first channels, whose sums are not stored.
+            const int go = n * g.K * g.OHW + y * P0.OW + ox;
 #pragma unroll
-            for (int e = 0; e < GU; ++e)
+            for (int e = 0; e < GU; ++e) {
+                const int k = k0 + (gk + e * 6) * 8;
+                const int o = in && k < g.K ? (go + k * g.OHW) * 4 : kSplitOOB;
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    gr_[e][i] = load1(rg, go, (e * 48 + i) * g.OHW * 4);
+                for (int i = 0; i < 8; ++i) gr_[e][i] = load1(rg, o, i * g.OHW * 4);
+            }
 #pragma unroll
             for (int e = 0; e < XU; ++e) {
                 const int Yx = Y0 + xrow[e], imx = P0.by_hs.div(Yx), nx = P0.by_ns.div(imx);
                 const int iy = Yx - imx * P0.Hs - P0.pady;
                 const int ix = (imx - nx * P0.NS) * P0.SW * g.st + xcol[e];
                 const bool ok = tile < tile1 && nx < g.imgs && (unsigned)iy < (unsigned)g.H &&
-                                (unsigned)ix < (unsigned)g.W;
+                                (unsigned)ix < (unsigned)g.W && xcg[e] >= 0;
                 const int o = ok ? (nx * g.C * g.HW + xcg[e] + iy * g.W + ix) * 4 : kSplitOOB;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) xr[e][i] = load1(rx, o, i * g.HW * 4);

@@ -32,9 +32,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t split_rsrc(const float *p, uin
 }
 // Floats at byte offset off (per lane) + so (the wave's): one, or eight in a
 // row.  A buffer load needs 4-byte alignment only, whatever its width.  The
-// range check of an unswizzled buffer counts both parts and does not wrap
-// (1024 bytes described, off 0..504: so = 768 returns the first 256 bytes' lanes
-// and zeros, so = 24000 zeros), so a channel or k past the end reads zero.
+// range check counts both parts (measured with 1024 bytes described and off
+// 0..504: so = 768 returns the first 256 bytes' lanes and zeros, so = 24000
+// zeros), so what lies past the operand's end reads zero.  off + so as unsigned
+// numbers stay below 2^32 in every call: operands end below 2^30; off lies in
+// the operand or is kSplitOOB; so lies in it, at most 31 k (31 channels) past it
+// or 7 channels past kSplitEnd, and below 2^31.
 __device__ __forceinline__ float load1(__amdgpu_buffer_rsrc_t r, int off, int so) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, so, 0));
 }
@@ -53,6 +56,7 @@ __device__ __forceinline__ void load8(__amdgpu_buffer_rsrc_t r, int off, int so,
 constexpr int kSchedNoVmem = 0x38f;
 // A byte offset beyond any operand: such a load returns zero.
 constexpr int kSplitOOB = (int)0x80000000;
+constexpr int kSplitEnd = 1 << 30;  // the end of the largest operand
 constexpr int kSplitFlush = 128;  // k summed on the matrix cores before the total takes them
 
 // One operand's tile of BI rows by BK k.  KC: the operand is contiguous

@@ -124,3 +124,32 @@ def test_split_dw(xs, ws, stride, pad):
     reach = np.zeros(ws[2:], bool)
     reach[max(0, pad - oh + 1):pad + 1, max(0, pad - ow + 1):pad + 1] = True
     assert np.array_equal(bad[3, 2], reach) and not np.delete(bad, 2, axis=1).any()
+
+
+def test_split_conv_large_planes():
+    """Channels far apart: a chunk after the two of 17 channels would end beyond 2^31 bytes, and
+    the tensors end just below 1 GiB.  Sampled outputs, corners and both passes."""
+    import torch
+    from katsu_amd import ops
+    xs, ws, hw = (1, 17, 3400, 3400), (20, 17, 3, 3), 3400
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    x = torch.randn(xs, generator=gen, device="cuda")
+    gy = torch.randn((1, 20, hw, hw), generator=gen, device="cuda")
+    w = torch.from_numpy(synth.he_normal(2, ws)).cuda()
+    rng = np.random.default_rng(4)
+    at = [tuple(p) for p in rng.integers(0, hw, (60, 2))] + [(0, 0), (hw - 1, hw - 1), (0, hw - 1)]
+
+    def check(got, inp, filt, what):
+        for y0, x0 in at:
+            r0, c0 = max(0, y0 - 1), max(0, x0 - 1)
+            patch = inp[0, :, r0:y0 + 2, c0:x0 + 2].double()
+            f = filt[:, :, r0 - y0 + 1:r0 - y0 + 1 + patch.shape[1],
+                     c0 - x0 + 1:c0 - x0 + 1 + patch.shape[2]].double()
+            ref = (patch * f).sum((1, 2, 3)).cpu().numpy()
+            sab = (patch.abs() * f.abs()).sum((1, 2, 3)).cpu().numpy()
+            assert_within(got[0, :, y0, x0].cpu().numpy(), ref, sab, inp.shape[1] * 9,
+                          f"{what} at {y0}, {x0}")
+
+    check(ops.conv2d_forward(x, w, 1, 1), x, w, "y")
+    check(ops.conv2d_backward_data(gy, w, xs, 1, 1), gy, w.transpose(0, 1).flip(2, 3), "dX")
