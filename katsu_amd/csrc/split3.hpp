@@ -27,9 +27,11 @@
 // Accumulation.  The instruction adds its 16 products to the accumulator
 // aligned to the largest term and keeps 2 bits below the accumulator's last
 // one (measured: 1 + 32 * 2^-26 is exact, 1 + 32 * 2^-27 is 1): a long sum
-// would lose the tails of terms of one sign.  The kernels therefore sum runs of
-// kFlush reduction steps from zero and add each run to a float32 total with
-// an ordinary addition, so that terms and accumulator stay near in size.
+// would lose the tails of terms of one sign.  The kernels therefore sum short
+// runs from zero (128 k of a GEMM, at most 9 steps or 144 products of a
+// convolution, 64 pixels of a filter gradient) and add each run to a float32
+// total with an ordinary addition, so that terms and accumulator stay near in
+// size.
 //
 // Non-finite values: Inf - Inf in the split, or a value that overflows when it
 // is scaled or rounded to bf16, makes the sum NaN or Inf; a finite sum holds

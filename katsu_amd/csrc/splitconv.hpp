@@ -100,6 +100,7 @@ struct SplitConv {
     static constexpr int kWBytes = 6 * kWPlane;
     static constexpr int kUnits = 2 * BM * TG;         // 8-channel groups of a filter stage
     static constexpr int WU = (kUnits + kThreads - 1) / kThreads;
+    static constexpr int kRun = 9;  // matrix steps of 16 products summed before the total takes them
     static constexpr int kSum = WPX * WKG * FM * FN * 4096;  // the waves' sums
 
     static constexpr int plane(int slots) { return slots * 16 + 32; }
@@ -207,10 +208,22 @@ struct SplitConv {
         };
 
         const int chunks = (g.CI + 15) / 16, groups = (taps + TG - 1) / TG;
+        // The total takes the sums after whole chunks, about every kSplitFlush
+        // products, and between groups of taps before a wave passes kRun steps.
         const int flush_every = max(1, kSplitFlush / (16 * taps));
+        auto flush = [&] {
+#pragma unroll
+            for (int a = 0; a < FM; ++a)
+#pragma unroll
+                for (int b = 0; b < FN; ++b) {
+                    tot[a][b] += acc[a][b];
+                    acc[a][b] = floatx16{};
+                }
+        };
+        auto steps = [](int n) { return (n + WKG - 1) / WKG; };
         load_x(0);
         load_w(0, 0);
-        int flush_in = flush_every;
+        int flush_in = flush_every, run = 0;
         for (int c = 0; c < chunks; ++c) {
 #pragma unroll
             for (int e = 0; e < XU; ++e) {
@@ -262,17 +275,19 @@ struct SplitConv {
                                 acc[a][b] = mfma32(af[a][kSplitA[q]], bf[b][kSplitB[q]], acc[a][b]);
                 }
                 __syncthreads();
+                if (!last) {
+                    run += steps(nt);
+                    if (run + steps(min(TG, taps - t0 - TG)) > kRun) {
+                        run = 0;
+                        flush();
+                    }
+                }
             }
             if (--flush_in == 0 || c + 1 == chunks) {
                 flush_in = flush_every;
-#pragma unroll
-                for (int a = 0; a < FM; ++a)
-#pragma unroll
-                    for (int b = 0; b < FN; ++b) {
-                        tot[a][b] += acc[a][b];
-                        acc[a][b] = floatx16{};
-                    }
+                flush();
             }
+            run = 0;
         }
 
         // The wave groups' sums, added in order by the first group.

@@ -23,6 +23,11 @@ def _scaled(seed, shape, s):
     return (synth.uniform(seed, shape).astype(np.float64) * s).astype(np.float32)
 
 
+def _rel(got, ref):
+    """Error in the 2-norm."""
+    return float(np.linalg.norm(got.cpu().numpy() - ref) / np.linalg.norm(ref))
+
+
 def _pick(t, at):
     v = t.cpu().numpy()
     return np.array([v[i] for i in at])
@@ -64,3 +69,31 @@ def test_dw_operand_scales(s, t):
     dw = ops.conv2d_backward_filter(_dev(x), _dev(gy), ws, stride, pad)
     at = random_samples(ws, 200, 5)
     assert_within(_pick(dw, at), *sample_dw(x, gy, ws, stride, pad, at), xs[0] * oh * ow, "dW")
+
+
+# Sums of long runs on the matrix cores lose the tails of terms of one sign, so the kernels
+# break them: the error must not grow with the filter.  Bounds on the 2-norm, in roundings of
+# the total (2^-24 = 6e-8): 2.5 for terms of one sign, 6 for signed ones, whose result is
+# smaller than its terms.  Sums over all taps of a chunk showed 3.0e-7 and 4.3e-7.
+LONG_FILTERS = [  # x, w, stride, pad
+    ((4, 12, 45, 52), (128, 12, 7, 7), 1, 3),    # 49 taps in one chunk, one wave for all
+    ((2, 16, 40, 40), (64, 16, 15, 15), 1, 7),   # 225 taps
+    ((8, 15, 33, 31), (40, 15, 5, 5), 1, 2),
+    ((2, 32, 56, 56), (64, 32, 3, 3), 1, 1),
+]
+
+
+@pytest.mark.parametrize("xs,ws,stride,pad", LONG_FILTERS)
+@pytest.mark.parametrize("one_signed", [True, False])
+def test_conv_error_does_not_grow_with_the_filter(xs, ws, stride, pad, one_signed):
+    from katsu_amd import ops
+    from tests.test_gpu_split_conv import _ref
+    oh, ow = ((xs[i + 2] + 2 * pad - ws[i + 2]) // stride + 1 for i in (0, 1))
+    x, w, gy = (synth.uniform(s, sh) for s, sh in ((1, xs), (2, ws), (3, (xs[0], ws[0], oh, ow))))
+    if one_signed:
+        x, w, gy = np.abs(x), np.abs(w), np.abs(gy)
+    y, dx = _ref(x, w, gy, stride, pad)
+    lim = 1.5e-7 if one_signed else 3.5e-7
+    err_y = _rel(ops.conv2d_forward(_dev(x), _dev(w), stride, pad), y)
+    err_dx = _rel(ops.conv2d_backward_data(_dev(gy), _dev(w), xs, stride, pad), dx)
+    assert max(err_y, err_dx) < lim, (err_y, err_dx)
