@@ -1050,9 +1050,12 @@ bool dx_phases(const ConvDims &d, const float *gy, const float *w, float *dx, fl
 
 // The stride-2 data gradient as a stride-1 problem over super-pixels (see
 // direct.hpp, WMODE 2): input G, 4C output channels, super-filter offsets
-// [amin, amax] per axis.
+// [amin, amax] per axis.  SF: rows and columns of the super-filter, 4 with few
+// channels or 2.
+template <int SF>
 bool dx_superpixel(const ConvDims &d, const float *gy, const float *w, float *dx, float beta,
                    hipStream_t st, int *rc) {
+    static_assert(SF == 2 || SF == 4, "super-filter");
     if (d.st != 2) return false;
     auto range = [&](int64_t R, int64_t *lo, int64_t *hi) {
         *lo = INT64_MAX;
@@ -1078,12 +1081,13 @@ bool dx_superpixel(const ConvDims &d, const float *gy, const float *w, float *dx
     P.g_bmin = bmin;
     P.fh = d.H;
     P.fw = d.W;
-    if (P.R == DxSp4::R && P.S == DxSp4::S && P.CO <= 16) return try_direct<DxSp4, 2, 1>(P, st, rc);
-    if (P.R == DxSp2::R && P.S == DxSp2::S) {
+    if (P.R != SF || P.S != SF) return false;
+    if constexpr (SF == 4) {
+        return P.CO <= 16 && try_direct<DxSp4, 2, 1>(P, st, rc);
+    } else {
         if (P.OW <= 16 && try_direct<DxSp2R, 2, 1>(P, st, rc)) return true;
         return try_direct<DxSp2, 2, 1>(P, st, rc);
     }
-    return false;
 }
 
 // The data gradient as a forward problem (stride 1 only): G convolved with
@@ -2038,6 +2042,80 @@ int fwd_cfg(const float *x, const float *w, float *y, const ConvDims &d, hipStre
     return run<C>(p, tiles_n * p.tiles_m, st);
 }
 
+// The generic engine's tile for the forward pass, the largest that still gives
+// every CU a block (rows x pixels), and for the data gradient.
+enum class Tile { S, M, L, T64, T32 };
+
+Tile fwd_tile(const ConvDims &d) {
+    const int64_t px = d.npix_out;
+    if (d.K <= 16) return Tile::S;
+    if (d.K > 64 && cdiv(d.K, 128) * cdiv(px, 128) >= kMinDirectBlocks) return Tile::L;
+    if (cdiv(d.K, 64) * cdiv(px, 128) >= kMinDirectBlocks) return Tile::M;
+    if (cdiv(d.K, 64) * cdiv(px, 64) >= kMinDirectBlocks) return Tile::T64;
+    return Tile::T32;
+}
+
+Tile dx_tile(const ConvDims &d) { return d.C <= 16 ? Tile::S : d.C <= 64 ? Tile::M : Tile::L; }
+
+// The times of the float32 kernels in microseconds, for the choice between them
+// and the split ones (split.hpp): of the generic engine a fixed part, the k-steps
+// of the longest block or of all blocks on a CU, whichever takes longer, and one
+// part per block on a CU.  (Of the data gradient's phases the longest counts, as an
+// XCD holds a run of blocks, of one or two phases.)  Fitted to the layers of
+// split.hip's estimate (6200 runs): nine in ten take 0.9 to 1.25 of it.
+struct IgemmUs { double launch, chain, step, block; };
+struct TileUs { int bm, bn, bk; IgemmUs fwd, dx; };
+constexpr TileUs kTileUs[] = {  // in Tile's order
+    {16, 256, 16, {2.9, 2.04, 1.21, 0.53}, {4.1, 2.02, 1.28, 0.48}},
+    {64, 128, 16, {5.4, 2.08, 1.015, 0.49}, {5.3, 1.63, 1.15, 0.88}},
+    {128, 128, 16, {7.3, 2.98, 1.63, 1.9}, {7.9, 2.12, 1.87, 2.96}},
+    {64, 64, 16, {3.1, 1.21, 0.56, 0.82}, {}},
+    {32, 32, 32, {2.5, 0.785, 0.48, 0.47}, {}}};
+
+struct IgemmWork {
+    const TileUs &t;
+    int64_t longest = 0, blocks = 0;
+    void add(int64_t rows, int64_t px, int64_t kred) {
+        longest = std::max(longest, cdiv(kred, t.bk));
+        blocks += cdiv(rows, t.bm) * cdiv(px, t.bn);
+    }
+    double us(const IgemmUs &u) const {
+        const double per_cu = (double)blocks / 256.;
+        return u.launch + std::max(u.chain, u.step * per_cu) * (double)longest + u.block * per_cu;
+    }
+};
+
+double igemm_fwd_us(const ConvDims &d) {
+    IgemmWork wk{kTileUs[(int)fwd_tile(d)]};
+    wk.add(d.K, d.npix_out, d.CRS);
+    return wk.us(wk.t.fwd);
+}
+
+double igemm_dx_us(const ConvDims &d) {
+    IgemmWork wk{kTileUs[(int)dx_tile(d)]};
+    const int n = std::min(d.st, 2);  // the split kernels take strides 1 and 2
+    for (int py = 0; py < n; ++py)
+        for (int px = 0; px < n; ++px) {
+            const int64_t r0 = (py + d.pad) % n, s0 = (px + d.pad) % n;
+            wk.add(d.C, (int64_t)d.N * cdiv(d.H - py, n) * cdiv(d.W - px, n),
+                   d.K * cdiv(d.R - r0, n) * cdiv(d.S - s0, n));
+        }
+    return wk.us(wk.t.dx);
+}
+
+// The stride-1 forward's direct plan and its time: per block on a CU a fixed part
+// and one of 8 input channels (40 runs, nine in ten within 0.93 to 1.1).
+bool direct_fwd_s1_plan(const DirectFwdProblem &P, DirectFwdPlan *pl) {
+    if (P.st != 1 || P.CO < FwdV::KT) return false;
+    return fwd_pitch8(P.OW)
+               ? direct_fwd_plan<FwdVP::KT, FwdVP::F, FwdVP::CB, FwdVP::R, FwdVP::S, FwdVP::ROWS,
+                                 FwdVP::PITCH, 0>(P, pl)
+               : direct_fwd_plan<KATSU_FWD_VARIANT, 0>(P, pl);
+}
+double direct_fwd_us(const DirectFwdPlan &pl, int64_t C) {
+    return 4.4 + (double)cdiv(pl.blocks, kMinDirectBlocks) * (3.7 + 3.4 * (double)cdiv(C, 8));
+}
+
 int conv_fwd_dev(const float *x, const float *w, float *y, const katsu_conv_geom *g,
                  hipStream_t st) {
     ConvDims d;
@@ -2052,20 +2130,20 @@ int conv_fwd_dev(const float *x, const float *w, float *y, const katsu_conv_geom
         if (stem_fwd(x, w, y, d, st, &rc)) return rc;
         if (pw_ok(d)) return pw_fwd(x, w, y, d, st);
         if (tiny_ok(d)) return tiny_fwd(x, w, y, d, st);
-        // Stride 2 reads four input pixels per output one: with a few channels
-        // and pixels the generic engine's smaller steps are ahead (32 -> 24
-        // channels, 3x3, 119 x 119: 11.1 / 13.4 us).
-        const bool small = d.st == 2 && d.C <= 32 && d.npix_out <= 4096;
-        if (!small && split_conv_fwd(x, w, y, split_layer(d), st, &rc)) return rc;
+        DirectFwdPlan pl;
+        const double below =
+            direct_fwd_s1_plan(P, &pl) ? direct_fwd_us(pl, d.C) : igemm_fwd_us(d);
+        if (split_conv_fwd(x, w, y, split_layer(d), below, st, &rc) == SplitRun::kLaunched)
+            return rc;
         if (direct_fwd<0>(P, st, &rc)) return rc;
     }
-    // The largest tile that still gives every CU a block (rows x pixels).
-    const int64_t px = d.npix_out;
-    if (d.K <= 16) return fwd_cfg<CfgS>(x, w, y, d, st);
-    if (d.K > 64 && cdiv(d.K, 128) * cdiv(px, 128) >= kMinDirectBlocks)
-        return fwd_cfg<CfgL>(x, w, y, d, st);
-    if (cdiv(d.K, 64) * cdiv(px, 128) >= kMinDirectBlocks) return fwd_cfg<CfgM>(x, w, y, d, st);
-    if (cdiv(d.K, 64) * cdiv(px, 64) >= kMinDirectBlocks) return fwd_cfg<Cfg64>(x, w, y, d, st);
+    switch (fwd_tile(d)) {
+        case Tile::S: return fwd_cfg<CfgS>(x, w, y, d, st);
+        case Tile::M: return fwd_cfg<CfgM>(x, w, y, d, st);
+        case Tile::L: return fwd_cfg<CfgL>(x, w, y, d, st);
+        case Tile::T64: return fwd_cfg<Cfg64>(x, w, y, d, st);
+        case Tile::T32: break;
+    }
     return fwd_cfg<Cfg32>(x, w, y, d, st);
 }
 
@@ -2220,14 +2298,23 @@ int conv_bwd_data_dev(const float *gy, const float *w, float *dx, const katsu_co
     // A layer whose one-call backward shares a launch with its dW keeps the
     // float32 kernel of that launch, so that both ways give the same bits.
     if (dx_as_forward(d, gy, w, dx, beta, &P) && direct_fwd<1>(P, st, &rc)) return rc;
-    if (!pw_ok(d) && !tiny_ok(d) && split_conv_dx(gy, w, dx, split_layer(d), beta, st, &rc))
-        return rc;
-    if (dx_superpixel(d, gy, w, dx, beta, st, &rc)) return rc;
+    // The 4x4 super-filter with few channels fills 16-row tiles where the split
+    // kernels' 32 rows hold 4 channels (25 images of 4 channels, 205 x 205, 7x7: 103
+    // / 366 us).  The 2x2 one loses to them on 42 of 44 layers (by 1.4 in the middle)
+    // and stays for the operands they don't take.
+    if (dx_superpixel<4>(d, gy, w, dx, beta, st, &rc)) return rc;
+    SplitRun run = SplitRun::kUnfit;
+    if (!pw_ok(d) && !tiny_ok(d))
+        run = split_conv_dx(gy, w, dx, split_layer(d), beta, igemm_dx_us(d), st, &rc);
+    if (run == SplitRun::kLaunched) return rc;
+    if (run == SplitRun::kUnfit && dx_superpixel<2>(d, gy, w, dx, beta, st, &rc)) return rc;
     if (pw_ok(d)) return pw_dx(gy, w, dx, d, beta, st);
     if (tiny_ok(d)) return tiny_dx(gy, w, dx, d, beta, st);
-    if (d.C <= 16) return dx_cfg<CfgS>(gy, w, dx, d, beta, st);
-    if (d.C <= 64) return dx_cfg<CfgM>(gy, w, dx, d, beta, st);
-    return dx_cfg<CfgL>(gy, w, dx, d, beta, st);
+    switch (dx_tile(d)) {
+        case Tile::S: return dx_cfg<CfgS>(gy, w, dx, d, beta, st);
+        case Tile::M: return dx_cfg<CfgM>(gy, w, dx, d, beta, st);
+        default: return dx_cfg<CfgL>(gy, w, dx, d, beta, st);
+    }
 }
 
 // ---------------------------------------------------------------------------

@@ -251,17 +251,27 @@ void phase_set(SplitPhase *p, const PhaseTiles &t, int imgs, int st) {
 // 512 channels at 7 x 7, 256 -> 256 at 14 x 14 and 64 -> 64 at 56 x 56, batch
 // 16-32).  The small tiles wait for their loads, the large ones approach the
 // matrix rate, so a layer takes the largest tile that still fills the GPU.
+//
+// us: the whole launch in microseconds, for the choice between these kernels and
+// the float32 ones: a fixed part, and per round of blocks one of the block, of a
+// block whose stores are two pixels apart, of each chunk, of each chunk's tap, and
+// of each chunk's input pixels per thread.  Of several phases the largest counts:
+// an XCD holds a run of tiles, of one or two phases.  Fitted to 7600 runs over
+// layers of 1 to 512 channels, filters of 1 to 9, both passes and strides: nine in
+// ten take 0.87 to 1.2 of it.
 struct ConvShape {
     int FM, FN, WPX, WKG, TG;
     double alone, shared;
+    struct { double launch, block, apart, chunk, tap, slot; } us;
     constexpr int bm() const { return 32 * FM; }
     constexpr int bn() const { return 32 * FN * WPX; }
     constexpr int threads() const { return 64 * WPX * WKG; }
 };
-constexpr ConvShape kConvShapes[] = {{2, 2, 4, 1, 5, 9500, 14500},
-                                     {1, 2, 4, 1, 9, 5600, 7700},
-                                     {1, 1, 4, 2, 9, 3200, 4500},
-                                     {1, 1, 2, 4, 9, 2800, 3800}};
+constexpr ConvShape kConvShapes[] = {
+    {2, 2, 4, 1, 5, 9500, 14500, {4.4, 4.0, 2.8, 1.14, 0.78, 0}},
+    {1, 2, 4, 1, 9, 5600, 7700, {3.3, 3.0, 0.6, 1.24, 0.41, 0}},
+    {1, 1, 4, 2, 9, 3200, 4500, {2.2, 2.6, 1.0, 0.33, 0.227, 1.47}},
+    {1, 1, 2, 4, 9, 2800, 3800, {0, 4.15, 1.4, 0.35, 0.176, 1.53}}};
 constexpr int kNumConvShapes = 4;
 constexpr int kMaxXU = 8;
 
@@ -278,8 +288,9 @@ int conv_lds(int c, int slots) {
     return conv_lds_of(c, slots, std::make_integer_sequence<int, kNumConvShapes>());
 }
 
-// The block shape of least estimated time, -1 if none takes the problem.
-int conv_pick(const SplitConvArgs &g) {
+// The block shape of least estimated time, -1 if none takes the problem; *us:
+// the launch in microseconds.
+int conv_pick(const SplitConvArgs &g, double *us) {
     int best = -1;
     double t_best = 0;
     for (int c = 0; c < kNumConvShapes; ++c) {
@@ -287,6 +298,7 @@ int conv_pick(const SplitConvArgs &g) {
         const int64_t tm = cdiv(g.CO, s.bm()), chunks = cdiv(g.CI, 16);
         int64_t blocks = 0, slots = 0;
         double taps = 0;
+        int most_taps = 0;
         bool ok = true;
         for (int i = 0; i < g.nphases; ++i) {
             const SplitPhase &p = g.ph[i];
@@ -298,6 +310,7 @@ int conv_pick(const SplitConvArgs &g) {
             blocks += t.tiles * tm;
             // Below five taps a chunk is bound by its loads.
             taps += (double)t.tiles * tm * std::max(5, p.Ru * p.Su);
+            most_taps = std::max(most_taps, p.Ru * p.Su);
         }
         if (!ok || 2 * slots > kMaxXU * s.threads() || blocks >= (int64_t)1 << 31) continue;
         const int lds = conv_lds(c, (int)slots);
@@ -307,11 +320,15 @@ int conv_pick(const SplitConvArgs &g) {
         const int64_t per_cu = lds <= kMaxLds / 2 ? 2 : 1;
         const int64_t full = blocks / (kCUs * per_cu), rest = blocks - full * kCUs * per_cu;
         const double round = per_cu == 2 ? s.shared : s.alone;
-        const double t = ((double)full * round + (rest > kCUs ? s.shared : rest ? s.alone : 0.)) *
-                         (double)chunks * taps / (double)blocks / 9.;
+        const double rounds = (double)full * round + (rest > kCUs ? s.shared : rest ? s.alone : 0.);
+        const double t = rounds * (double)chunks * taps / (double)blocks / 9.;
         if (best < 0 || t < t_best) {
             best = c;
             t_best = t;
+            const double chunk = s.us.chunk + s.us.tap * most_taps +
+                                 s.us.slot * (double)slots / s.threads();
+            *us = s.us.launch + rounds / s.alone * (s.us.block + (g.osx > 1 ? s.us.apart : 0.) +
+                                                    (double)chunks * chunk);
         }
     }
     return best;
@@ -342,14 +359,22 @@ int conv_go(SplitConvArgs &g, hipStream_t st) {
     return conv_launch<S.FM, S.FN, S.WPX, S.WKG, S.TG, kMaxXU>(g, blocks, st);
 }
 
-bool conv_run(SplitConvArgs &g, hipStream_t st, int *rc) {
-    switch (conv_pick(g)) {
-        case 0: *rc = conv_go<0>(g, st); return true;
-        case 1: *rc = conv_go<1>(g, st); return true;
-        case 2: *rc = conv_go<2>(g, st); return true;
-        case 3: *rc = conv_go<3>(g, st); return true;
-        default: return false;
+// below: the time another kernel would take, in microseconds.
+SplitRun conv_run(SplitConvArgs &g, double below, hipStream_t st, int *rc) {
+    double us = 0;
+    const int shape = conv_pick(g, &us);
+    if (shape < 0) return SplitRun::kUnfit;
+    // Both estimates are off by a tenth: with 3% to the other kernel's advantage
+    // 1 layer in 100 is slower by more than a twentieth than with it, and 1 in 60
+    // slower than here (without: 1 in 75 and 1 in 90).
+    if (us * 1.03 >= below) return SplitRun::kSlower;
+    switch (shape) {
+        case 0: *rc = conv_go<0>(g, st); break;
+        case 1: *rc = conv_go<1>(g, st); break;
+        case 2: *rc = conv_go<2>(g, st); break;
+        default: *rc = conv_go<3>(g, st); break;
     }
+    return SplitRun::kLaunched;
 }
 
 bool layer_args(const SplitLayer &l, SplitConvArgs *g) {
@@ -480,25 +505,25 @@ bool dx_args(const SplitLayer &l, SplitConvArgs *out) {
 
 }  // namespace
 
-bool split_conv_fwd(const float *x, const float *w, float *y, const SplitLayer &l, hipStream_t st,
-                    int *rc) {
+SplitRun split_conv_fwd(const float *x, const float *w, float *y, const SplitLayer &l,
+                        double below, hipStream_t st, int *rc) {
     SplitConvArgs g;
-    if (!fwd_args(l, &g)) return false;
+    if (!fwd_args(l, &g)) return SplitRun::kUnfit;
     g.in = x;
     g.w = w;
     g.out = y;
-    return conv_run(g, st, rc);
+    return conv_run(g, below, st, rc);
 }
 
-bool split_conv_dx(const float *gy, const float *w, float *dx, const SplitLayer &l, float beta,
-                   hipStream_t st, int *rc) {
+SplitRun split_conv_dx(const float *gy, const float *w, float *dx, const SplitLayer &l, float beta,
+                       double below, hipStream_t st, int *rc) {
     SplitConvArgs g;
-    if (!dx_args(l, &g)) return false;
+    if (!dx_args(l, &g)) return SplitRun::kUnfit;
     g.in = gy;
     g.w = w;
     g.out = dx;
     g.beta = beta;
-    return conv_run(g, st, rc);
+    return conv_run(g, below, st, rc);
 }
 
 namespace {
