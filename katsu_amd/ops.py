@@ -15,13 +15,11 @@ from ._abi import check, geometry, lib
 # A small call's time is its host side (a pass of four 48 x 56 products and
 # fills took 31 us, the GPU 14): the stream as the raw handle torch's own
 # launchers read (0.3 us, against 2.9 through torch.cuda.current_stream()'s
-# Stream object), pointers as integers, which the argtypes convert.
-_raw_stream = torch._C._cuda_getCurrentRawStream
-_device = torch._C._cuda_getDevice
-
-
+# Stream object), pointers as integers, which the argtypes convert.  The names
+# are looked up per call: a torch without a GPU build does not have them.
 def _stream():
-    return _raw_stream(_device())
+    c = torch._C
+    return c._cuda_getCurrentRawStream(c._cuda_getDevice())
 
 
 def _p(t):
