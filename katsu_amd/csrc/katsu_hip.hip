@@ -2426,7 +2426,8 @@ DwPlan dw_plan_any(const ConvDims &d) {
     DirectFwdPlan xp;
     if (dp.ok && (d.st == 2 || (dx_as_forward(d, nullptr, nullptr, nullptr, 0.f, &P) &&
                                 P.CO >= FwdV::KT &&
-                                direct_fwd_plan<KATSU_FWD_VARIANT, 1>(P, &xp)))) {
+                                direct_fwd_plan<KATSU_FWD_VARIANT, 1>(P, &xp) &&
+                                dw_variant_fusable(dp.variant, d.st)))) {
         DwPlan pl{};
         pl.ws_bytes = dp.ws_bytes;
         pl.direct = dp;

@@ -45,3 +45,29 @@ def test_conv_route(op, xs, ws, stride, pad, kernel):
     got = out.cpu().numpy()
     vals, sabs = ref(a, w, stride, pad, at)
     assert_within(np.array([got[i] for i in at]), vals, sabs, kred, op)
+
+
+DW_ROUTES = [  # x, w, stride, pad, split or not, with the times of the float32 and the split kernel
+    ((30, 96, 20, 20), (128, 96, 3, 3), 1, 1, True),
+    ((14, 96, 144, 80), (64, 96, 1, 1), 1, 1, False),  # one tap of nine: 47 / 88 us
+    ((30, 16, 109, 119), (64, 16, 2, 2), 1, 0, False),  # 52 / 94 us
+    ((3, 427, 9, 9), (384, 427, 5, 5), 1, 2, False),   # 243 pixels: 35 / 79 us
+    ((5, 303, 10, 10), (234, 303, 7, 7), 1, 3, False),  # 500 pixels: 61 / 88 us
+]
+
+
+@pytest.mark.parametrize("xs,ws,stride,pad,split", DW_ROUTES)
+def test_dw_route(xs, ws, stride, pad, split):
+    import torch
+    from katsu_amd import ops
+    from tests.parity import sample_dw
+    oh, ow = ((xs[i + 2] + 2 * pad - ws[i + 2]) // stride + 1 for i in (0, 1))
+    x, gy = synth.uniform(1, xs), synth.normal(3, (xs[0], ws[0], oh, ow))
+    xd, gd = torch.from_numpy(x).cuda(), torch.from_numpy(gy).cuda()
+    out = torch.empty(ws, device="cuda")
+    names = kernels(lambda: ops.conv2d_backward_filter(xd, gd, ws, stride, pad, out=out))
+    assert ("split_dw_kernel" in names) == split, names
+    at = random_samples(ws, 100, 5) + [(0, 0, 0, 0), tuple(d - 1 for d in ws)]
+    got = out.cpu().numpy()
+    vals, sabs = sample_dw(x, gy, ws, stride, pad, at)
+    assert_within(np.array([got[i] for i in at]), vals, sabs, xs[0] * oh * ow, "dW")
