@@ -158,9 +158,9 @@ def test_filter_gradient_is_deterministic(dev):
 def test_baseline_layers_small_batch(name, batch, dev):
     """The BASELINE layers' channel and kernel shapes at a batch of 1 or 2,
     full oracle comparison with a random upstream gradient (all-ones would
-    hide a flipped kernel).  At these batches configs 3 and 4a take the
-    generic engine (too few tiles for the direct kernels); the production
-    kernels are the next test's."""
+    hide a flipped kernel).  At these batches configs 3 and 4a take the split
+    kernels and the generic engine (too few tiles for the direct kernels); the
+    production kernels are the next test's."""
     c = dict(synth.CONV_CONFIGS[name])
     c["x"] = (batch,) + c["x"][1:]
     x, w = synth.conv_inputs(c)
@@ -174,13 +174,14 @@ def test_baseline_layers_small_batch(name, batch, dev):
 _ROWS40 = dict(x=(32, 64, 40, 40), w=(64, 64, 3, 3), stride=1, pad=1, law="u11")
 
 
-@pytest.mark.parametrize("name,batch", [("c3_resnet", 9), ("c4a_down3x3", 16),
+@pytest.mark.parametrize("name,batch", [("c3_resnet", 10), ("c3_resnet", 9), ("c4a_down3x3", 16),
                                         ("c5_stem", 9), ("c4b_down1x1", 32),
                                         ("rows40", 32)])
 def test_production_kernels_full_parity(name, batch, dev):
     """The kernels the BASELINE configurations run (the direct 3x3 kernels of
     configs 3 and 4a and their one-launch backward, the stem's kernels, the
-    1x1 kernels) at the smallest batch where the planner picks them: every
+    1x1 kernels) at the smallest batch where the planner picks them, and config
+    3 one image below it, on the split kernels: every
     element of y, dX and dW, from the separate calls and from the one-call
     backward, against the oracle on finite random data."""
     import torch

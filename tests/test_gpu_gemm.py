@@ -61,11 +61,12 @@ def test_matmul_and_vjp_parity(m, k, n, dev):
     assert_within(db.cpu().numpy(), db_ref, aa.T @ ag + np.abs(db0), m + 1, "dB")
 
 
-# (m, n, k): unaligned (the generic engine), then multiples of 4 (the
-# dedicated GEMM: 64-tiles with split-K, a long split-K reduction, 128-tiles
-# with edge tiles, 32-tiles at 512 deep), then the register-direct GEMM
-# (64-tiles, K = 1024 in four wave quarters; tiles in patches of four tile
-# rows, or in column order when the tile rows are not a multiple of four).
+# (m, n, k): unaligned, then multiples of 4: most on the split GEMM of the bf16
+# matrix cores; 128 x 96 x 2048 (a long sum of few tiles: split-K) and 512^3
+# (32-tiles) on the dedicated float32 GEMM; 1024 x 512 and 192 x 2752 x 1024 on
+# the register-direct GEMM (64-tiles, K = 1024 in four wave quarters; tiles in
+# patches of four tile rows, or in column order when the tile rows are not a
+# multiple of four).
 @pytest.mark.parametrize("m,n,k", [(70, 45, 131), (72, 44, 132), (128, 96, 2048),
                                    (516, 260, 68), (1024, 512, 1024), (512, 512, 512),
                                    (256, 640, 512), (192, 2752, 1024)])

@@ -13,8 +13,8 @@ Inf, -Inf and NaN are planted in x, w and G at border taps (a corner of the
 filter, the first and last rows and columns of the images) and in the
 interior.  Batches are chosen so each layer takes the kernels the planner
 uses at the BASELINE size (the direct halo kernels need enough tiles to fill
-the chip): config 3 at N = 9, config 4a at N = 16, the stem at N = 9; a
-config-3 layer at N = 2 takes the generic engine, config 4b the 1x1 kernels
+the chip): config 3 at N = 10, config 4a at N = 16, the stem at N = 9; a
+config-3 layer at N = 2 or 9 takes the split kernels, config 4b the 1x1 kernels
 and config 1 the few-channel kernels."""
 import numpy as np
 import pytest
@@ -93,8 +93,9 @@ def _run_all(x, w, g, st, p, dev):
 
 
 CASES = [
-    ("c3_resnet", 9),     # direct forward, stride-1 dX, one-launch backward
-    ("c3_resnet", 2),     # the generic engine (too few tiles for the direct kernels)
+    ("c3_resnet", 10),    # stride-1 dX and dW on the direct kernels, one-launch backward
+    ("c3_resnet", 9),     # all three passes on the split kernels
+    ("c3_resnet", 2),     # forward and dX on the split kernels
     ("c4a_down3x3", 16),  # stride-2 forward, phase-form dX, stride-2 dW
     ("c4b_down1x1", 4),   # 1x1 kernels (no padding)
     ("c5_stem", 9),       # stem forward, dW and rolling-row dX
@@ -134,7 +135,7 @@ def test_nonfinite_inputs_match_oracle(name, batch, dev):
 
 def test_nonfinite_host_entry_points(dev):
     """The drop-in host-pointer entry points on a config-3 layer with planted
-    non-finite values (direct kernels, N = 9)."""
+    non-finite values (split kernels, N = 9)."""
     from katsu_amd import host
     c = dict(synth.CONV_CONFIGS["c3_resnet"])
     c["x"] = (9,) + c["x"][1:]

@@ -70,13 +70,14 @@ def _operands(m, k, n):
 
 
 # (m, k, n) and the kernels they take:
-#   37 x 41 x 29       the generic engine (dimensions not multiples of 4)
+#   37 x 41 x 29       not multiples of 4: the split GEMM; dA, whose sums are 29
+#                      long, on the generic engine
 #   512^3              32 x 32 tiles; the VJP's dA and dB blocks in one launch
 #   64 x 1000 x 64     64-tiles with K split six ways + the fixed-order reduce;
-#                      one-launch VJP on 64-tiles
-#   1024 x 100 x 1024  64-tiles; the VJP's two products split K eight ways
+#                      split VJP
+#   1024 x 100 x 1024  split; the VJP's two products on 64-tiles, K split eight ways
 #   1024^3             the register-direct kernels (forward and one-launch VJP)
-#   2048 x 64 x 2048   128 x 128 tiles with edge tiles in K; split VJP
+#   2048 x 64 x 2048   split; the VJP's two products with K split
 SHAPES = [(37, 41, 29), (512, 512, 512), (64, 1000, 64), (1024, 100, 1024),
           (1024, 1024, 1024), (2048, 64, 2048)]
 

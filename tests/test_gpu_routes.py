@@ -1,6 +1,7 @@
-"""Which kernel a convolution takes on both sides of the split kernels' rule, and its values.
+"""Which kernel a convolution or a product takes on both sides of the split kernels' rules, and
+its values.
 
-The rule compares estimated times (csrc/split.hip, conv_run): few input channels fill a matrix
+The convolutions' rule compares estimated times (csrc/split.hip, conv_run): few input channels fill a matrix
 step of 16, and few output channels a tile of 32, too little to pay for six bf16 products."""
 import numpy as np
 import pytest
@@ -71,3 +72,48 @@ def test_dw_route(xs, ws, stride, pad, split):
     got = out.cpu().numpy()
     vals, sabs = sample_dw(x, gy, ws, stride, pad, at)
     assert_within(np.array([got[i] for i in at]), vals, sabs, xs[0] * oh * ow, "dW")
+
+
+def test_superpixel_2x2_beyond_1gib():
+    """A 3x3 stride-2 dX of 1 GiB, which the split kernels don't take: sampled outputs of the 2x2
+    super-pixel form."""
+    import torch
+    from katsu_amd import ops
+    xs, ws = (4700, 16, 60, 60), (20, 16, 3, 3)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(6)
+    gy = torch.randn((xs[0], ws[0], 29, 29), generator=gen, device="cuda")
+    w = synth.he_normal(2, ws)
+    wd, out = torch.from_numpy(w).cuda(), torch.empty(xs, device="cuda")
+    call = lambda: ops.conv2d_backward_data(gy, wd, xs, 2, 0, out=out)
+    assert kernels(call) == {"direct_fwd_kernel"}
+    for n in (0, 2345, 4699):
+        at = random_samples((1,) + xs[1:], 200, 5) + edge_samples((1,) + xs[1:])
+        vals, sabs = sample_dx(gy[n:n + 1].cpu().numpy(), w, (1,) + xs[1:], 2, 0, at)
+        got = out[n:n + 1].cpu().numpy()
+        assert_within(np.array([got[i] for i in at]), vals, sabs, ws[0] * 9, f"image {n}")
+
+
+GEMM_ROUTES = [  # m, k, n, kernel
+    (2052, 16, 2100, "gemm_kernel"),     # short sums: 128-tiles
+    (1000, 20, 1100, "gemm_kernel"),     # 64-tiles
+    (33, 31, 65, "igemm_kernel"),        # unaligned and short
+    (33, 32, 65, "split_gemm_kernel"),
+    (512, 512, 512, "gemm_kernel"),      # 32-tiles
+    (64, 904, 64, "gemm_kernel"),        # a long sum of few tiles: split over blocks
+    (64, 900, 64, "split_gemm_kernel"),
+    (1024, 1024, 1024, "gemm_rd_kernel"),
+    (2048, 32, 2048, "split_gemm_kernel"),
+]
+
+
+@pytest.mark.parametrize("m,k,n,kernel", GEMM_ROUTES)
+def test_gemm_route(m, k, n, kernel):
+    import torch
+    from katsu_amd import ops
+    a, b = synth.uniform(1, (m, k)), synth.uniform(2, (k, n))
+    ad, bd = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    out = torch.empty((m, n), device="cuda")
+    assert kernel in kernels(lambda: ops.gemm(ad, bd, m, n, k, out=out))
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    assert_within(out.cpu().numpy(), a64 @ b64, np.abs(a64) @ np.abs(b64), k, "C")

@@ -3,24 +3,25 @@
 Layers at the edges of their tiles: images that share a tile and images that do not, strips of
 wide rows, channel counts off the chunks of 16 and the tiles of 32 and 64, filters of fewer and
 more taps than are staged together, both strides and all their phases, padding beyond the
-filter.  Bound: that of a float32 dot product in any order (tests/parity.py); what the split
+filter.  Each test asserts that the split kernel is the one that runs.  Bound: that of a float32 dot product in any order (tests/parity.py); what the split
 leaves out is at most a quarter of the rounding it counts per product."""
 import numpy as np
 import pytest
 
 from katsu_amd import synth
 from tests.parity import assert_within
+from tests.routes import kernels
 
 pytestmark = pytest.mark.gpu
 
 LAYERS = [  # x, w, stride, pad
-    ((3, 17, 7, 7), (33, 17, 3, 3), 1, 1),       # images share tiles, tails of every kind
+    ((3, 81, 7, 7), (33, 81, 3, 3), 1, 1),       # images share tiles, tails of every kind
     ((2, 40, 29, 31), (70, 40, 3, 3), 1, 1),
-    ((1, 16, 20, 65), (32, 16, 3, 3), 1, 1),     # two strips of 33 and 32 columns
-    ((2, 9, 12, 130), (20, 9, 5, 5), 1, 2),      # three strips, 25 taps
+    ((1, 80, 20, 65), (32, 80, 3, 3), 1, 1),     # two strips of 33 and 32 columns
+    ((2, 41, 12, 130), (20, 41, 5, 5), 1, 2),    # three strips, 25 taps
     ((32, 32, 40, 48), (64, 32, 3, 3), 1, 1),    # 64 x 256 and 32 x 256 tiles
     ((9, 24, 56, 56), (96, 24, 2, 3), 1, 0),     # rectangular filter, no padding
-    ((2, 20, 13, 11), (18, 20, 3, 3), 1, 4),     # padding beyond the filter
+    ((2, 120, 13, 11), (18, 120, 3, 3), 1, 4),   # padding beyond the filter
     ((2, 50, 33, 47), (30, 50, 7, 7), 2, 3),     # stride 2: four phases of 16, 12, 12, 9 taps
     ((3, 36, 30, 29), (41, 36, 5, 5), 2, 2),
     ((2, 48, 21, 70), (40, 48, 4, 4), 2, 1),     # even filter
@@ -46,9 +47,13 @@ def test_split_conv(xs, ws, stride, pad):
     y, dx = _ref(x, w, gy, stride, pad)
     sy, sdx = _ref(np.abs(x), np.abs(w), np.abs(gy), stride, pad)
     kf, kb = ws[1] * ws[2] * ws[3], ws[0] * ws[2] * ws[3]
-    got = ops.conv2d_forward(dev(x), dev(w), stride, pad)
+    xd, wd, gd = dev(x), dev(w), dev(gy)
+    assert kernels(lambda: ops.conv2d_forward(xd, wd, stride, pad)) == {"split_conv_kernel"}
+    assert kernels(lambda: ops.conv2d_backward_data(gd, wd, xs, stride,
+                                                    pad)) == {"split_conv_kernel"}
+    got = ops.conv2d_forward(xd, wd, stride, pad)
     assert_within(got.cpu().numpy(), y, sy, kf, "y")
-    got = ops.conv2d_backward_data(dev(gy), dev(w), xs, stride, pad)
+    got = ops.conv2d_backward_data(gd, wd, xs, stride, pad)
     assert_within(got.cpu().numpy(), dx, sdx, kb, "dX")
     old = synth.uniform(4, xs)
     acc = dev(old)
@@ -85,11 +90,39 @@ def test_split_conv_nonfinite(xs, ws, stride, pad):
     assert np.isfinite(ref).any() and not np.isfinite(ref).all()
 
 
+@pytest.mark.parametrize("xs,ws,stride,pad", [LAYERS[0], LAYERS[3], LAYERS[8]])
+def test_split_dx_nonfinite(xs, ws, stride, pad):
+    """The same of the data gradient, at stride 2 in all four phases."""
+    import torch
+    from katsu_amd import ops
+    w = synth.he_normal(2, ws)
+    oh, ow = ((xs[i + 2] + 2 * pad - ws[i + 2]) // stride + 1 for i in (0, 1))
+    gy = synth.normal(3, (xs[0], ws[0], oh, ow))
+    gy[0, 0, 0, 0], gy[-1, 1, -1, -1], gy[0, -1, oh // 2, ow // 2] = np.inf, -np.inf, np.nan
+    w[2, 3, 0, 0] = np.inf
+    dx = ops.conv2d_backward_data(torch.from_numpy(gy).cuda(), torch.from_numpy(w).cuda(), xs,
+                                  stride, pad).cpu().numpy()
+    gd, wd = gy.astype(np.float64), w.astype(np.float64)
+    ref = np.zeros(xs)
+    with np.errstate(invalid="ignore"):
+        for oy in range(oh):
+            for ox in range(ow):
+                y0, x0 = oy * stride - pad, ox * stride - pad
+                r = slice(max(0, -y0), min(ws[2], xs[2] - y0))
+                s = slice(max(0, -x0), min(ws[3], xs[3] - x0))
+                ref[:, :, y0 + r.start:y0 + r.stop, x0 + s.start:x0 + s.stop] += (
+                    gd[:, :, oy, ox][:, :, None, None, None] * wd[None, :, :, r, s]).sum(1)
+    for mask in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(mask(dx), mask(ref))
+    assert np.isfinite(ref).any() and not np.isfinite(ref).all()
+
+
 DW_LAYERS = [  # x, w, stride, pad: 1.5 GFLOP or more, so that the split kernel takes them
     ((30, 96, 20, 20), (128, 96, 3, 3), 1, 1),   # whole images
     ((40, 160, 14, 14), (130, 160, 3, 3), 1, 1),  # tiles across images, channel tail
     ((3, 40, 90, 130), (60, 40, 5, 5), 1, 2),    # strips, three sets of taps
     ((8, 64, 30, 33), (64, 64, 7, 7), 1, 3),
+    ((40, 64, 199, 15), (64, 64, 3, 2), 2, 1),   # stride 2: few columns, whose rows fit the LDS
 ]
 
 
@@ -108,7 +141,10 @@ def test_split_dw(xs, ws, stride, pad):
     pick = lambda t: np.array([t[i] for i in at])
     ref, sabs = sample_dw(x, gy, ws, stride, pad, at)
     n = xs[0] * oh * ow
-    dw = ops.conv2d_backward_filter(dev(x), dev(gy), ws, stride, pad)
+    xd, gd = dev(x), dev(gy)
+    assert "split_dw_kernel" in kernels(
+        lambda: ops.conv2d_backward_filter(xd, gd, ws, stride, pad))
+    dw = ops.conv2d_backward_filter(xd, gd, ws, stride, pad)
     assert_within(pick(dw.cpu().numpy()), ref, sabs, n, "dW")
     _, dw2 = ops.conv2d_backward(dev(x), dev(w), dev(gy), stride, pad)
     assert torch.equal(dw, dw2)
@@ -122,7 +158,10 @@ def test_split_dw(xs, ws, stride, pad):
     got = ops.conv2d_backward_filter(dev(x), dev(gy), ws, stride, pad).cpu().numpy()
     bad = ~np.isfinite(got)
     reach = np.zeros(ws[2:], bool)
-    reach[max(0, pad - oh + 1):pad + 1, max(0, pad - ow + 1):pad + 1] = True
+    for i in range(ws[2]):
+        for j in range(ws[3]):
+            oy, ox = (pad - i) / stride, (pad - j) / stride
+            reach[i, j] = oy in range(oh) and ox in range(ow)
     assert np.array_equal(bad[3, 2], reach) and not np.delete(bad, 2, axis=1).any()
 
 

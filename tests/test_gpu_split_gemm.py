@@ -2,14 +2,16 @@
 
 Shapes at the edges of each of its tiles (32, 64, 128 and 256 x 128), with sums that end
 inside a matrix step, a stage and a run of 128 k, from pointers that are only 4-byte aligned;
-forward, both VJP products in their one launch, and beta = 1.  Bound: that of a float32 dot
+forward, both VJP products (in one launch or two), and beta = 1.  Bound: that of a float32 dot
 product in any order (tests/parity.py); the split's own error, at most 2^-26 of each product, is
-a quarter of the rounding it counts per product.  Integers are exact in all six bf16 products."""
+a quarter of the rounding it counts per product.  Whole numbers of 12 by 4 bits are exact in two
+of the six bf16 products (tests/test_gpu_split_precision.py has numbers for each of them)."""
 import numpy as np
 import pytest
 
 from katsu_amd import synth
 from tests.parity import assert_within
+from tests.routes import kernels
 
 pytestmark = pytest.mark.gpu
 
@@ -38,7 +40,7 @@ def test_split_gemm(m, k, n, shift):
     ad, bd, gd = (_dev(v, shift) for v in (a, b, g))
     a64, b64, g64 = (v.astype(np.float64) for v in (a, b, g))
     c = _dev(np.full((m, n), np.nan, np.float32), shift)
-    ops.gemm(ad, bd, m, n, k, out=c)
+    assert kernels(lambda: ops.gemm(ad, bd, m, n, k, out=c)) == {"split_gemm_kernel"}
     assert_within(c.cpu().numpy(), a64 @ b64, np.abs(a64) @ np.abs(b64), k, "C")
     da0, db0 = synth.uniform(14, (m, k)), synth.uniform(15, (k, n))
     da, db = _dev(da0, shift), _dev(db0, shift)

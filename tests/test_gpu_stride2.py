@@ -5,11 +5,12 @@ parity), and on rows of at most 16 output pixels the row-fragment tiles;
 cases cover 14- and 15-pixel rows and input channel counts with and without
 16-byte weight rows.  Data gradient: a 3x3, padding-1 layer with at least 16
 input channels takes the phase form (every MFMA a real tap, all four output
-phases of a channel block in one block); other stride-2 layers take the
-super-pixel form (a stride-1 convolution of G over 2x2 pixel blocks, then
-scattered back), except the stem's own channel counts (3 in, 64 out), which
-take the rolling-row kernel (each output row summed over its four G rows in
-the accumulators).  Phase-form cases cover odd image sizes (a super-pixel's
+phases of a channel block in one block); the stem's own channel counts (3 in,
+64 out, 7x7) take the rolling-row kernel (each output row summed over its four
+G rows in the accumulators); other stride-2 layers take the split kernels, the
+generic engine or, 7x7 ones of few channels and many pixels, the super-pixel
+form (a stride-1 convolution of G over 2x2 pixel blocks, then scattered back:
+tests/test_gpu_routes.py).  Phase-form cases cover odd image sizes (a super-pixel's
 second row or column outside the image), channel counts off the 16-channel
 blocks and stages, rows of exactly 16 super-pixels, tiles of 5 rows with a
 short last tile, and beta = 1.  Shapes are chosen so the planner takes these
@@ -52,7 +53,7 @@ def test_forward_stride2(xs, ws, dev):
                                      ((32, 64, 27, 27), (128, 64, 3, 3), 1),
                                      ((32, 64, 28, 28), (128, 64, 3, 3), 0)])
 def test_data_gradient_3x3(xs, ws, p, dev):
-    """Padding 1 takes the phase form, padding 0 the super-pixel form."""
+    """Padding 1 takes the phase form, padding 0 the split kernels."""
     import torch
 
     from katsu_amd import ops
@@ -150,8 +151,8 @@ def test_stride2_small_image_all_passes(xs, ws, dev):
 
 
 # 7x7 stride-2 padding-3 data gradient of layers with at most 4 input
-# channels (stem-like), full oracle comparison: odd sizes clip the last
-# super-pixel's second row and column, an odd K, C = 1 and C = 4, beta = 1.
+# channels (stem-like), full oracle comparison: odd sizes, an odd K, C = 1 and
+# C = 4, beta = 1 (too few pixels for the super-pixel form: the split kernels).
 STEM_DX_CASES = [
     ((32, 3, 99, 101), (25, 3, 7, 7)),
     ((64, 4, 64, 72), (16, 4, 7, 7)),
