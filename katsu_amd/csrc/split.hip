@@ -601,14 +601,16 @@ size_t split_dw_bytes(const SplitLayer &l) {
     // GFLOP: 31 us against 21; 128 -> 128 at 28 x 28, batch 8, 1.85 GFLOP: 38
     // against 45).  So do half-empty tiles of 64 x 32 channels and 9 taps (13 -> 15
     // channels 5x5: 266 against 205; 45 -> 83 channels 5x5: forward + backward 155
-    // against 145; 128 -> 64 channels 1x1, padded: 155 against 62), and so few
-    // pixels that a block's partial sums are most of its work (243 pixels, 427 ->
-    // 384 channels 5x5: 79 against 35; 500: 88 against 61; 1024: 61 against 73).
+    // against 145; 128 -> 64 channels 1x1, padded: 155 against 62).  With
+    // several sets of taps and few pixels the partial sums and their reduction
+    // are most of the work (243 pixels, 427 -> 384 channels 5x5: 79 against 35; of
+    // 170 such layers the middle one breaks even at 1000 pixels with 5x5 filters
+    // and near 1700 with 7x7; with 3x3 ones all of 169 gain, down to 150 pixels).
     const int taps = l.R * l.S;
     const double flops = 2. * l.N * l.OH * l.OW * l.K * l.C * taps;
     const double fill = (double)l.K * l.C * taps /
                         ((double)cdiv(l.K, 64) * 64 * cdiv(l.C, 32) * 32 * cdiv(taps, 9) * 9);
-    if (flops < 1.5e9 || fill < 0.5 || (int64_t)l.N * l.OH * l.OW < 1000) return 0;
+    if (flops < 1.5e9 || fill < 0.5 || (taps > 9 && (int64_t)l.N * l.OH * l.OW < 1500)) return 0;
     return dw_args(l, &g) ? (size_t)(g.runs * g.run_stride) * sizeof(float) : 0;
 }
 

@@ -50,6 +50,8 @@ def test_conv_route(op, xs, ws, stride, pad, kernel):
 
 DW_ROUTES = [  # x, w, stride, pad, split or not, with the times of the float32 and the split kernel
     ((30, 96, 20, 20), (128, 96, 3, 3), 1, 1, True),
+    ((16, 512, 7, 7), (512, 512, 3, 3), 1, 1, True),   # 784 pixels: 112 / 59 us
+    ((31, 64, 7, 7), (320, 64, 5, 5), 1, 2, True),     # 1519 pixels
     ((14, 96, 144, 80), (64, 96, 1, 1), 1, 1, False),  # one tap of nine: 47 / 88 us
     ((30, 16, 109, 119), (64, 16, 2, 2), 1, 0, False),  # 52 / 94 us
     ((3, 427, 9, 9), (384, 427, 5, 5), 1, 2, False),   # 243 pixels: 35 / 79 us
