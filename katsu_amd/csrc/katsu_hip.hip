@@ -455,8 +455,9 @@ int gemm_rd_launch(const GemmArgs &g, hipStream_t st) {
 //     equal near K = 900 (64 x 1000 x 64: 10.9 / 9.4 us; 16 x 1024 x 128: 8.6 /
 //     10.2).
 // Elsewhere the split ones win, by 1.1-1.7x on aligned problems (2048^3: 139 /
-// 109 us, 4096^3: 1041 / 640 us) and by more on others (1001 x 1531 x 777:
-// 59 / 26 us).  Operands of 1 GiB and more stay on the generic engine.
+// 109 us, 4096^3: 1063 / 647 us) and by more on others (1001 x 1531 x 777:
+// 58 / 27 us).  Of 1300 random aligned products 44 are slower here by a twentieth;
+// times fitted to both kernels would have chosen no better.  Operands of 1 GiB and more stay on the generic engine.
 constexpr int64_t kSplitMinK = 32, kSplitMaxKFewTiles = 900;
 
 bool gemm_on_split(const SplitProblem &p) {

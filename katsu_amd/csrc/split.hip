@@ -105,7 +105,8 @@ int64_t tiles_of(const SplitProblem &p, int T) {
 }
 
 // The tile of least estimated time, in ns: a round is one block on every CU,
-// and costs a fixed part and a part per k.  Fitted to measured times: 256 x 128
+// and costs a fixed part and a part per k.  Fitted to times measured before the
+// operands were scaled (split3.hpp), which adds 2-8% to all of them: 256 x 128
 // tiles 4096^3 in 627 us (2 rounds) and 4096 x 16 x 4096 in 24; 128-tiles
 // 2048^3 in 111 us (1 round); 64-tiles 1024^3 in 20.4 us (1 round) and 2048^3
 // in 126 (4); 32-tiles 300^3 in 6.2 us and 64 x 8192 x 64 in 50 (1 round each).

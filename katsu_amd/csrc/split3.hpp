@@ -56,8 +56,8 @@ constexpr float kSplitUnscale = 0x1p-32f;  // of a sum
 
 // Eight floats as three vectors of eight bf16: 13 vector instructions a pair.
 // (The differences as two-term bf16 products on the packed pair are exact too
-// and take 7, but run slower beside the matrix instructions: 4096^3 in 687
-// against 632 us.)
+// and take 4 fewer, but run slower beside the matrix instructions: 4096^3 in 687
+// against 632 us, both without the two that scale; 647 with them.)
 __device__ __forceinline__ void split3(const float (&x)[8], uintx4 (&p)[3]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

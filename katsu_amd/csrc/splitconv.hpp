@@ -18,10 +18,11 @@
 // meet in LDS, in order, at the end.
 //
 // What it runs at (batch 32, one MI355X, forward then dX; float32 kernels before):
-// 64 -> 64 channels 3x3 at 56 x 56 65 (74) us forward, 256 -> 256 at 14 x 14 75
-// (186) and 73 (314), 45 -> 83 5x5 at 37 x 51, batch 7, 40 (96) and 51 (216).
-// What bounds it: the small tiles their loads (one chunk in flight), the large
-// ones the split and the LDS beside the matrix instructions.
+// 64 -> 64 channels 3x3 at 56 x 56 61 (64) us forward, 256 -> 256 at 14 x 14 73
+// (178) and 72 (314), 45 -> 83 5x5 at 37 x 51, batch 7, 39 (90) and 53 (216).
+// What bounds it: waits, for the one chunk of loads in flight and at the barriers
+// (a third of the waves' cycles); the matrix cores are 20-31% busy, the other
+// vector instructions 19-34%, the LDS 15-27%, a quarter of it bank conflicts.
 //
 // Wide images are cut into strips of at most 64 columns, each treated as an
 // image of its own, to bound the rows' length in LDS.

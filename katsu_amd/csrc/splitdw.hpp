@@ -18,8 +18,8 @@
 // 128-byte lines, and split_dw_reduce adds them in order.
 //
 // Measured (one MI355X, the reduction included; float32 kernels before): 256 -> 256
-// channels 3x3 at 14 x 14, batch 32, 74 us (145); 512 -> 512 at 7 x 7, batch 16, 59
-// (115); 96 -> 96 5x5 at 56 x 56, batch 16, 325 (503).  Of the 78 us that 64 -> 64
+// channels 3x3 at 14 x 14, batch 32, 68 us (139); 512 -> 512 at 7 x 7, batch 16, 58
+// (111); 96 -> 96 5x5 at 56 x 56, batch 16, 297 (529).  Of the 78 us that 64 -> 64
 // at 56 x 56 took, 32 are matrix instructions and their reads, 14 waits for
 // loads, 6 the split, and the rest start, partial sums and their reduction.
 #pragma once
