@@ -553,6 +553,12 @@ int gemm_dev(const float *a, const float *b, float *c, size_t m, size_t n, size_
     return gemm_dispatch<Cfg32>(a, b, c, m, n, k, ta, tb, beta, st);
 }
 
+// Of a VJP with one product on the split kernels and one on the float32 ones, up
+// to this many float32 blocks both stay in one float32 launch: the launch saved
+// outweighs the faster product (240 x 384 x 16: 8.3 us, in two launches 10.3; 32 x
+// 1504 x 12: 6.0 / 8.7; but 400 x 56464 x 4, 2210 blocks: 78 / 55).
+constexpr int64_t kMixedVjpMaxBlocks = 256;
+
 // Matmul VJP (tensor.rs:418-445): da = beta_a*da + g b^T, then
 // db = beta_b*db + a^T g; a null da or db skips that product.  When both are
 // wanted, their buffers do not overlap, and both plan the same unsplit tile,
@@ -573,56 +579,53 @@ int matmul_vjp_dev(const float *a, const float *b, const float *g, float *da, fl
         const SplitProblem pa{g, b, da, M, K, N, 0, 1, beta_a}, pb{a, g, db, K, N, M, 1, 0, beta_b};
         const bool sa = gemm_on_split(pa), sb = gemm_on_split(pb);
         if (sa && sb) return split_gemm_vjp(pa, pb, st);
-        // One on each side: two launches, below.
-        if (!sa && !sb) {
-            GemmArgs ra, rb;
-            if (gemm_rd_plan(g, b, da, M, K, N, 0, 1, beta_a, &ra) &&
-                gemm_rd_plan(a, g, db, K, N, M, 1, 0, beta_b, &rb) &&
-                (ra.tiles_m * ra.tiles_n) % 8 == 0) {
-                ra.c = da;
-                rb.c = db;
-                const int nb0 = ra.tiles_m * ra.tiles_n, nb1 = rb.tiles_m * rb.tiles_n;
-                if (KATSU_GEMM_RD_VJP_PAIR && nb0 == nb1) {
-                    // One block per tile index: its dA tile, then its dB tile.
-                    constexpr auto pk =
-                        gemm_rd_vjp_pair_kernel<kRdVjpKs, kRdVjpNkb, KATSU_GEMM_RD_VJP_D>;
-                    constexpr size_t lds = kRdVjpKs * 64 * 64 * 4;
-                    const int rc = lds_optin<pk>(lds);
-                    if (rc != KATSU_OK) return rc;
-                    pk<<<dim3((unsigned)nb0), dim3(64 * kRdVjpKs), lds, st>>>(ra, rb);
-                    return launch_status();
-                }
-                constexpr auto kern =
-                    gemm_rd_vjp_kernel<kRdVjpKs, kRdVjpNkb, KATSU_GEMM_RD_VJP_D, KATSU_GEMM_RD_VJP_OCC>;
+        GemmArgs ra, rb;
+        if (!sa && !sb && gemm_rd_plan(g, b, da, M, K, N, 0, 1, beta_a, &ra) &&
+            gemm_rd_plan(a, g, db, K, N, M, 1, 0, beta_b, &rb) &&
+            (ra.tiles_m * ra.tiles_n) % 8 == 0) {
+            ra.c = da;
+            rb.c = db;
+            const int nb0 = ra.tiles_m * ra.tiles_n, nb1 = rb.tiles_m * rb.tiles_n;
+            if (KATSU_GEMM_RD_VJP_PAIR && nb0 == nb1) {
+                // One block per tile index: its dA tile, then its dB tile.
+                constexpr auto pk =
+                    gemm_rd_vjp_pair_kernel<kRdVjpKs, kRdVjpNkb, KATSU_GEMM_RD_VJP_D>;
                 constexpr size_t lds = kRdVjpKs * 64 * 64 * 4;
-                const int rc = lds_optin<kern>(lds);
+                const int rc = lds_optin<pk>(lds);
                 if (rc != KATSU_OK) return rc;
-                kern<<<dim3((unsigned)(nb0 + nb1)), dim3(64 * kRdVjpKs), lds, st>>>(ra, rb, nb0);
+                pk<<<dim3((unsigned)nb0), dim3(64 * kRdVjpKs), lds, st>>>(ra, rb);
                 return launch_status();
             }
-            GemmFastPlan fa, fb;
-            if (gemm_fast_plan(g, b, da, M, K, N, 0, 1, beta_a, &fa) &&
-                gemm_fast_plan(a, g, db, K, N, M, 1, 0, beta_b, &fb) && fa.T == fb.T &&
-                fa.splits == 1 && fb.splits == 1 && fa.blocks % 8 == 0 &&
-                fa.blocks + fb.blocks <= kI32Max) {
-                fa.g.c = da;
-                fb.g.c = db;
-                fa.g.split_stride = fb.g.split_stride = 0;
-                // Wave groups by the combined grid (two blocks per CU from the
-                // pair where each alone would take two groups): the k-sum order
-                // can then differ from the separate launches', within the f32
-                // bound and the same on every call.
-                const bool two = fa.blocks + fb.blocks < KATSU_GEMM_WG2_BELOW;
-                const int64_t b0 = fa.blocks, b1 = fb.blocks;
-                if (fa.T == 128)
-                    return two ? gemm_vjp_launch<128, 128, 16, 2>(fa.g, fb.g, b0, b1, st)
-                               : gemm_vjp_launch<128, 128, 16, 1>(fa.g, fb.g, b0, b1, st);
-                if (fa.T == 64)
-                    return two ? gemm_vjp_launch<64, 64, KATSU_GEMM_BK64, 2>(fa.g, fb.g, b0, b1, st)
-                               : gemm_vjp_launch<64, 64, KATSU_GEMM_BK64, 1>(fa.g, fb.g, b0, b1, st);
-                return two ? gemm_vjp_launch<32, 32, KATSU_GEMM_BK32, 2>(fa.g, fb.g, b0, b1, st)
-                           : gemm_vjp_launch<32, 32, KATSU_GEMM_BK32, 1>(fa.g, fb.g, b0, b1, st);
-            }
+            constexpr auto kern =
+                gemm_rd_vjp_kernel<kRdVjpKs, kRdVjpNkb, KATSU_GEMM_RD_VJP_D, KATSU_GEMM_RD_VJP_OCC>;
+            constexpr size_t lds = kRdVjpKs * 64 * 64 * 4;
+            const int rc = lds_optin<kern>(lds);
+            if (rc != KATSU_OK) return rc;
+            kern<<<dim3((unsigned)(nb0 + nb1)), dim3(64 * kRdVjpKs), lds, st>>>(ra, rb, nb0);
+            return launch_status();
+        }
+        GemmFastPlan fa, fb;
+        if (gemm_fast_plan(g, b, da, M, K, N, 0, 1, beta_a, &fa) &&
+            gemm_fast_plan(a, g, db, K, N, M, 1, 0, beta_b, &fb) && fa.T == fb.T &&
+            fa.splits == 1 && fb.splits == 1 && fa.blocks % 8 == 0 &&
+            fa.blocks + fb.blocks <= ((sa || sb) ? kMixedVjpMaxBlocks : kI32Max)) {
+            fa.g.c = da;
+            fb.g.c = db;
+            fa.g.split_stride = fb.g.split_stride = 0;
+            // Wave groups by the combined grid (two blocks per CU from the
+            // pair where each alone would take two groups): the k-sum order
+            // can then differ from the separate launches', within the f32
+            // bound and the same on every call.
+            const bool two = fa.blocks + fb.blocks < KATSU_GEMM_WG2_BELOW;
+            const int64_t b0 = fa.blocks, b1 = fb.blocks;
+            if (fa.T == 128)
+                return two ? gemm_vjp_launch<128, 128, 16, 2>(fa.g, fb.g, b0, b1, st)
+                           : gemm_vjp_launch<128, 128, 16, 1>(fa.g, fb.g, b0, b1, st);
+            if (fa.T == 64)
+                return two ? gemm_vjp_launch<64, 64, KATSU_GEMM_BK64, 2>(fa.g, fb.g, b0, b1, st)
+                           : gemm_vjp_launch<64, 64, KATSU_GEMM_BK64, 1>(fa.g, fb.g, b0, b1, st);
+            return two ? gemm_vjp_launch<32, 32, KATSU_GEMM_BK32, 2>(fa.g, fb.g, b0, b1, st)
+                       : gemm_vjp_launch<32, 32, KATSU_GEMM_BK32, 1>(fa.g, fb.g, b0, b1, st);
         }
     }
     int rc = KATSU_OK;
